@@ -8,7 +8,9 @@
 // calc_1Dto1D.cu:62-65, calc_3Dto3D.cu:43-137).
 //
 // Two forms of each lookup:
-//   * LIT  : the reference expression restated literally (fmod, IEEE division).
+//   * LIT  : any increment.  The reference's fmod and divisions, decided from
+//            the exact quotient and remainder by an fma (quot_rem), with the
+//            divisions themselves only where a decision is within rounding.
 //   * POW2 : used when every increment is a power of two.  Then x / inc and
 //            x * (1/inc) are the same real number, hence round identically,
 //            and fmod(x, inc) / inc == s - trunc(s) with s = x * (1/inc)
@@ -47,56 +49,69 @@ __device__ __forceinline__ int mul24(int a, int b) {
 }
 __device__ __forceinline__ double dmax(double a, double b) { return __builtin_fmax(a, b); }
 
-// fmod(x, y) for y > 0, exact (the IEEE remainder with the sign of x).
-// q = trunc(fl(x/y)) is the true quotient or one more (fl rounded up across
-// an integer); x - q*y is then r or r - y, both representable, so the fma is
-// exact, and the fix-up adds y back exactly.  |x/y| >= 2^53 only happens for
-// unclamped type II / 1D coordinates whose cell is clamped anyway.
-__device__ __forceinline__ double fmod_exact(double x, double y) {
-  double q = __builtin_trunc(x / y);
-  double r = __builtin_fma(-q, y, x);
-  if (x >= 0.0) {
-    if (r < 0.0) r = r + y;
-  } else {
-    if (r > 0.0) r = r - y;
+// The exact quotient and remainder of x >= 0 by inc: returns k = floor(x / inc)
+// and r = x - k inc = fmod(x, inc), without a division.  k0 = trunc(x * rinc)
+// (rinc the rounded reciprocal) is k or off by one: x * rinc is within 2^-52
+// relative of x / inc, and k counts only below 2^24 (a larger one is clamped
+// by the caller).  x - k0 inc is then r, r - inc or r + inc; the fma gives the
+// first two exactly (multiples of the smaller ulp, no larger than inc) and
+// rounds the last, if at all, without crossing inc, so its sign against 0 and
+// inc tells the case and the remainder is formed again with the right k.
+// The lookup is bound by VALU issue, and an IEEE FP64 division is about a
+// dozen instructions: with fmod, the index and the in-box coordinate each
+// dividing (three per axis), calc_T on MI355X took 277 us for 640 x 480
+// points (2D type I), 470 us for 10^6 points (1D, 50 cells) and 562 us for
+// 491 520 points (3D type I, with the remap); this way 175, 274 and 331 us.
+__device__ __forceinline__ double quot_rem(double x, double inc, double rinc, double& r) {
+  double k = __builtin_trunc(x * rinc);
+  r = __builtin_fma(-k, inc, x);
+  if ((r < 0.0) | (r >= inc)) {  // rare: x within rounding of a multiple of inc
+    k = r < 0.0 ? k - 1.0 : k + 1.0;
+    r = __builtin_fma(-k, inc, x);
   }
-  return r;
+  return k;
 }
-
-// calc_2Dto2D.cu:20-22
-__device__ __forceinline__ int mymin(int a, double b) { return !(b < a) ? a : (int)__builtin_round(b); }
 
 // One axis of the type II / 1D lookup:
 //   round(min(nC-1, max(0, (p - fmod(p, inc)) / inc)))
+// p - fmod(p, inc) is trunc(p / inc) multiples of inc, and its rounded
+// quotient by inc is within 1/2 of that count, so the result is the count
+// clamped to [0, nC-1]; fmod of +-inf or NaN is NaN, which max(0, NaN) turns
+// into 0.
 template <bool POW2>
 __device__ __forceinline__ int axis_box(double p, int nC, double inc, double rinc) {
-  double q;
   if (POW2) {
-    // (p - fmod(p,inc))/inc == trunc(p/inc); fmod of +-inf or NaN is NaN,
-    // which max(0, NaN) turns into 0.
-    q = __builtin_isfinite(p) ? __builtin_trunc(p * rinc) : 0.0;
-  } else {
-    q = (p - fmod_exact(p, inc)) / inc;
+    const double q = __builtin_isfinite(p) ? __builtin_trunc(p * rinc) : 0.0;
+    return (int)__builtin_round(dmin((double)(nC - 1), dmax(0.0, q)));
   }
-  return (int)__builtin_round(dmin((double)(nC - 1), dmax(0.0, q)));
+  // k0 = trunc(q * rinc) is off by one at most next to a multiple of inc
+  // (quot_rem); a count past nC - 1 stays there whatever its remainder reads
+  const double q = dmax(0.0, p);
+  const double k0 = __builtin_trunc(q * rinc);
+  const double r = __builtin_fma(-k0, inc, q);
+  int k = (int)dmin((double)nC, k0);
+  k += r >= inc ? 1 : (r < 0.0 ? -1 : 0);
+  k = k > nC - 1 ? nC - 1 : k;
+  return __builtin_isfinite(p) ? k : 0;
 }
 
-// One clamped axis of the type I lookups: returns the box index (mymin of
-// (p0 - xmod)/inc) and the in-box coordinate xmod/inc.
+// One clamped axis of the type I lookups: the box index (mymin of
+// (p0 - xmod) / inc, calc_2Dto2D.cu:20-22) and the in-box coordinate: frac =
+// xmod / inc (POW2), or the remainder xmod itself, whose division the caller
+// puts off (simplex_frac).
 template <bool POW2>
 __device__ __forceinline__ int axis_simplex(double p0, int nC, double inc, double rinc, double& frac) {
+  int i;
   if (POW2) {
     // p0 >= 0 (clamped), so s >= 0: s - trunc(s) is exact and equals
     // fract(s) = s - floor(s) (one v_fract_f64), and (int)s truncates.
     const double s = p0 * rinc;
     frac = __builtin_amdgcn_fract(s);
-    const int i = (int)s;
-    return i < nC - 1 ? i : nC - 1;
+    i = (int)s;
   } else {
-    double m = fmod_exact(p0, inc);
-    frac = m / inc;
-    return mymin(nC - 1, (p0 - m) / inc);
+    i = (int)quot_rem(p0, inc, rinc, frac);
   }
+  return i < nC - 1 ? i : nC - 1;
 }
 
 template <bool POW2>
@@ -112,6 +127,27 @@ __device__ __forceinline__ int cell1(const double* p, const Geom& g) {
 }
 
 // ------------------------------------------------------------------ 2D
+// Triangle of the point with in-box coordinates x, y (0 top, 1 right, 2
+// bottom, 3 left): the reference's tests x < y and 1 - x < y.  Without POW2
+// x and y come as the exact remainders and the reference's are their rounded
+// quotients by inc.  The products with rinc are within 2^-52 + 2^-54 of
+// those, so where both differences exceed 2^-50 they decide the same; only
+// next to a diagonal are the quotients formed.
+template <bool POW2>
+__device__ __forceinline__ int triangle_of(double x, double y, const Geom& g) {
+  if (!POW2) {
+    const double xa = x * g.rinc_x, ya = y * g.rinc_y;
+    const double d1 = xa - ya, d2 = (1.0 - xa) - ya;
+    if (__builtin_fabs(d1) > 0x1p-50 & __builtin_fabs(d2) > 0x1p-50)
+      return (d1 < 0.0) ? ((d2 < 0.0) ? 2 : 3) : ((d2 < 0.0) ? 1 : 0);
+    x = x / g.inc_x;
+    y = y / g.inc_y;
+  }
+  const double omx = 1.0 - x;
+  if (x < y) return (omx < y) ? 2 : 3;
+  return (omx < y) ? 1 : 0;
+}
+
 // calc_2Dto2D.cu:38-153
 // FAST (POW2 type I only): when every lane of the wave is strictly inside
 // (0, top) on both axes, min(top, max(0, p)) is p, trunc(p / inc) <= nC - 1
@@ -171,27 +207,31 @@ __device__ __forceinline__ int cell2(const double* p, const Geom& g) {
   const bool left = px <= 0.0, right = px >= g.wall_x, up = py <= 0.0, down = py >= g.wall_y;
   if (left | right | up | down) {  // rare: outside the domain
     // the reference's rules, as selects on the four sides' tests
-    const double nC0 = (double)g.nC0, nC1 = (double)g.nC1;
-    const double sx = divinc<POW2>(px, g.inc_x, g.rinc_x), sy = divinc<POW2>(py, g.inc_y, g.rinc_y);
-    const double nx = divinc<POW2>(-px, g.inc_x, g.rinc_x), ny = divinc<POW2>(-py, g.inc_y, g.rinc_y);
-    const bool upL = up & (sy < sx), dnL = down & (sy - nC1 > nx);
-    const bool upR = up & (ny > sx - nC0), dnR = down & (sy - nC1 > sx - nC0);
+    bool upL = false, dnL = false, upR = false, dnR = false;
+    if (POW2 || ((left | right) & (up | down))) {  // (without POW2 four divisions: past a corner only)
+      const double nC0 = (double)g.nC0, nC1 = (double)g.nC1;
+      const double sx = divinc<POW2>(px, g.inc_x, g.rinc_x), sy = divinc<POW2>(py, g.inc_y, g.rinc_y);
+      const double nx = divinc<POW2>(-px, g.inc_x, g.rinc_x), ny = divinc<POW2>(-py, g.inc_y, g.rinc_y);
+      upL = up & (sy < sx);
+      dnL = down & (sy - nC1 > nx);
+      upR = up & (ny > sx - nC0);
+      dnR = down & (sy - nC1 > sx - nC0);
+    }
     const int tl = upL ? 0 : (dnL ? 2 : 3);
     const int tr = upR ? 0 : (dnR ? 2 : 1);
     const int tm = up ? 0 : 2;
     return c + (left ? tl : (right ? tr : tm));
   }
-  const double omx = 1.0 - x;
-  if (x < y) return c + ((omx < y) ? 2 : 3);
-  return c + ((omx < y) ? 1 : 0);
+  return c + triangle_of<POW2>(x, y, g);
 }
 
 // cell2's general type I path without branches: the inside and outside
 // classifications are both computed and one is selected, so a lane that is
 // alone in its wave (a single dependent chain, see lone_trips) pays no
 // branch and no strict-interior test.  Same result as cell2 for every point.
-template <bool POW2>
+// Power-of-two increments only (the others' divisions are better left out).
 __device__ __forceinline__ int cell2_flat(const double* p, const Geom& g) {
+  constexpr bool POW2 = true;
   const double px = p[0], py = p[1];
   const double p0 = dmin(g.top_x, dmax(0.0, px));
   const double p1 = dmin(g.top_y, dmax(0.0, py));
@@ -234,6 +274,20 @@ __device__ __forceinline__ int cell3(const double* p, const Geom& g) {
   int c = mul24(i + mul24(j, g.nC0) + mul24(k, mul24(g.nC1, g.nC0)), 5);
   // alternating orientation: flip when the parity of i + j + k is odd
   const bool tf = ((i + j + k) & 1) != 0;
+  if (!POW2) {
+    // the remainders' products with rinc decide unless one of the four planes
+    // is within their error (three coordinates of 2^-52 + 2^-54 and the sums'
+    // roundings, below 2^-48), as in triangle_of
+    const double xa = x * g.rinc_x, ya = y * g.rinc_y, za = z * g.rinc_z;
+    const double u = tf ? ya : xa, v = tf ? 1.0 - xa : ya;
+    const double d1 = za - u - v, d2 = u + v + za - 2.0, d3 = v - u - za, d4 = u - v - za;
+    if (__builtin_fabs(d1) > 0x1p-48 & __builtin_fabs(d2) > 0x1p-48 & __builtin_fabs(d3) > 0x1p-48 &
+        __builtin_fabs(d4) > 0x1p-48)
+      return c + (d1 > 0.0 ? 1 : (d2 > 0.0 ? 2 : (d3 > 0.0 ? 3 : (d4 > 0.0 ? 4 : 0))));
+    x = x / g.inc_x;
+    y = y / g.inc_y;
+    z = z / g.inc_z;
+  }
   if (tf) {
     const double tmp = x;
     x = y;

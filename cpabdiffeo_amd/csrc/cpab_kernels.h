@@ -357,7 +357,7 @@ __device__ __forceinline__ bool trip(double* p, int& c, int& k, const double*& r
 // consistent with (c, k).
 template <int DIM, int TESS, bool POW2>
 __device__ __forceinline__ int lone_cell(const double* y, const Geom& g) {
-  if (DIM == 2 && TESS == TESS_I) return cell2_flat<POW2>(y, g);
+  if (DIM == 2 && TESS == TESS_I && POW2) return cell2_flat(y, g);
   return cell_of<DIM, TESS, POW2>(y, g);
 }
 
