@@ -122,6 +122,16 @@ int make_geom(cpab_ctx* ctx, int dim, int tess, int nC0, int nC1, int nC2, doubl
   g->top_z = nC2 * ix - 0.0000000001;  // the reference clamps z with inc_x (calc_3Dto3D.cu:59)
   g->wall_x = nC0 * ix;
   g->wall_y = nC1 * iy;
+  // Margin of CellBounds in units of the increments: its functions of p / inc
+  // and the lookup's own coordinates are within 2^-50 of nC of their true
+  // values up to 16 boxes past the domain, and the lookup clamps points 1e-10
+  // inside the far walls.
+  double nmax = 1.0, rmax = 0.0;
+  for (int d = 0; d < dim; d++) {
+    nmax = n[d] > nmax ? n[d] : nmax;
+    rmax = 1.0 / inc[d] > rmax ? 1.0 / inc[d] : rmax;
+  }
+  g->eps = (nmax + 16.0) * 0x1p-46 + 2e-10 * rmax;
   // The type I clamps must leave a non-empty range, or the box index of a
   // clamped point would be negative.
   if (tess == TESS_I && !(g->top_x > 0.0 && g->top_y > 0.0 && (dim < 3 || g->top_z > 0.0)))
@@ -155,7 +165,6 @@ struct Shape {
   int64_t grid;
   size_t lds;
   bool use_lds;
-  bool fast;  // enough waves per SIMD to be throughput-bound: the FAST 2D lookup pays
 };
 
 Shape integrate_shape(const cpab_ctx* ctx, int64_t nPts, int nC, int ne, int ntables) {
@@ -172,7 +181,6 @@ Shape integrate_shape(const cpab_ctx* ctx, int64_t nPts, int nC, int ne, int nta
   const int64_t waves = (nPts + s.ptsPerWave - 1) / s.ptsPerWave;
   const int wpb = s.block / 64;
   s.grid = (waves + wpb - 1) / wpb;
-  s.fast = waves >= (int64_t)ctx->n_cu * 4 * 4;  // four waves per SIMD or more
   return s;
 }
 
@@ -208,16 +216,6 @@ template <int DIM, int TESS, bool POW2, bool LDS>
 int launch_integrate_t(cpab_ctx* ctx, int mode, const Shape& s, const double* pos0, double* out,
                        const double* Trels, const double* As, double h, int nT, int nS, int64_t nPts,
                        const Geom& g, int nC, int32_t* nfb, const PrepSrc& ps) {
-  if constexpr (DIM == 2 && TESS == TESS_I && POW2) {
-    if (mode == 0 && s.fast) {
-      auto k = k_integrate<DIM, TESS, POW2, LDS, 0, true>;
-      allow_lds(k, s.lds);
-      hipLaunchKernelGGL(k, dim3((unsigned)s.grid), dim3(s.block), s.lds, ctx->stream, pos0, out, Trels, As, h, nT,
-                         nS, nPts, g, nC, s.ptsPerWave, nfb, ps);
-      HIP_OK(ctx, hipGetLastError());
-      return CPAB_OK;
-    }
-  }
   if (mode == 0) {
     auto k = k_integrate<DIM, TESS, POW2, LDS, 0>;
     allow_lds(k, s.lds);

@@ -8,8 +8,8 @@
 // atomic per chunk; a block leaves when the queue is exhausted, so every
 // block ends).  A block keeps the tables of the instance it is working on in
 // LDS and reloads them only when a tile of another instance comes; the waves
-// of a block split the tile's points and integrate them with the lane-skewed
-// loop of k_integrate.  Per point the arithmetic is exactly calc_T's, so a
+// of a block split the tile's points and integrate them with
+// k_integrate's two phases (`advance`).  Per point the arithmetic is exactly calc_T's, so a
 // point gives the same bits batched or alone.
 #pragma once
 #include "cpab_kernels.h"
@@ -69,8 +69,8 @@ __global__ void k_batch_reset(unsigned int* queue) {
 // power of two up to 1 024 in 1D, 32 in 2D, 8 in 3D, at least 16 points a
 // bucket on average), buckets in row order, built in LDS by the whole block.
 // Neighbouring points flow alike and cross facets at about the same steps,
-// so a wave's lanes then need closer numbers of trips than for points in
-// input order.  Within a bucket the order follows the LDS atomics, which may
+// so a wave's lanes then need closer numbers of steps and redos than for
+// points in input order.  Within a bucket the order follows the LDS atomics, which may
 // differ from run to run: that changes which lane integrates a point and
 // when, never the point's result.
 constexpr int kBucketTileMax = 16384;  // the most points of a sorted tile (16-bit indices)
@@ -177,7 +177,7 @@ __global__ void __launch_bounds__(1024)
       const int64_t b = tl.begin + (int64_t)w * per;
       const int64_t e = b + per < tl.end ? b + per : tl.end;
       if (b < e)
-        integrate_range<DIM, TESS, POW2, 0, true>(b, e, pos0, out, lds, lds + nC * NE, h, nT, nS, 0, g, nfb_out, 0,
+        integrate_range<DIM, TESS, POW2, 0>(b, e, pos0, out, lds, lds + nC * NE, h, nT, nS, 0, g, nfb_out, 0,
                                                   lord, tl.begin);
     }
   }
@@ -244,7 +244,7 @@ __global__ void __launch_bounds__(1024)
       const int64_t b = it.begin + (int64_t)w * per;
       const int64_t e = b + per < it.end ? b + per : it.end;
       if (b < e)
-        integrate_range<DIM, TESS, POW2, 0, false>(b, e, it.pos0, it.out, lds, lds + nC * NE, h, nT, nS, 0, g, nullptr,
+        integrate_range<DIM, TESS, POW2, 0>(b, e, it.pos0, it.out, lds, lds + nC * NE, h, nT, nS, 0, g, nullptr,
                                                    0, lord, it.begin);
     }
   }

@@ -37,6 +37,7 @@ struct Geom {
   double rinc_x, rinc_y, rinc_z;  // exact 1/inc (POW2 form only)
   double top_x, top_y, top_z;     // clamps nC0*inc_x-1e-10, nC1*inc_y-1e-10, nC2*inc_x-1e-10
   double wall_x, wall_y;          // nC0*inc_x, nC1*inc_y (2D type I out-of-domain tests)
+  double eps;                     // margin of CellBounds, in increments
 };
 
 __device__ __forceinline__ double dmin(double a, double b) { return __builtin_fmin(a, b); }
@@ -154,11 +155,10 @@ __device__ __forceinline__ int triangle_of(double x, double y, const Geom& g) {
 // and no outside rule applies, so the lookup is done without the clamps,
 // the index mins and the min/max operand canonicalisations IEEE mode needs.
 // The test is wave-uniform: a wave with a lane on or past the boundary (or
-// NaN) runs the general lookup only.  Measured on MI355X the gain depends
-// on the launch: 256 registration chains +14-17 %, one chain with deep
-// speculation +1-2 %, the 512x512 calc_T +3 %, the 1 024-instance batch
-// +1.5 %; but a 65536-point calc_T -28 % and the serving mix's work items
-// -5 %.  So each launch chooses it.
+// NaN) runs the general lookup only.  Measured on MI355X: 256 registration
+// chains +14-17 %, one chain with deep speculation +1-2 %, calc_T's redo
+// phase +0-3 %; but one chain one step per launch -15 %, so a registration
+// launch chooses it.
 template <int TESS, bool POW2, bool FAST = false, bool EARLY = true>
 __device__ __forceinline__ int cell2(const double* p, const Geom& g) {
   if (TESS == TESS_II) {
@@ -170,9 +170,9 @@ __device__ __forceinline__ int cell2(const double* p, const Geom& g) {
     // The interior form's cell.  EARLY: formed before the test that allows
     // it, so that the test's scalar chain and branch are off the cell's
     // critical path (a lane outside gets a value that is not used; measured
-    // on MI355X: the 512 x 512 calc_T -1.5 %, one registration chain +1.2 %,
-    // the batch -5.5 %, but 256 registration chains one step per launch 2 %
-    // slower, so those launches form it after the test).
+    // on MI355X: one registration chain +1.2 %, but 256 registration chains
+    // one step per launch 2 % slower, so those launches form it after the
+    // test).
     const uint64_t ex = __builtin_amdgcn_read_exec();
     if (EARLY) {
       const double sx = px * g.rinc_x, sy = py * g.rinc_y;  // > 0 inside: fract as in axis_simplex

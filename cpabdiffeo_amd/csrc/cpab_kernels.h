@@ -8,13 +8,12 @@
 //                  tables live in LDS.  The reference runs every step as
 //                  "Trel proposal, and on a cell change nStepsODE RK2
 //                  substeps", which in SIMT form idles 63 lanes of a wave
-//                  while one lane does its ten substeps.  Here every loop trip
-//                  of a lane is ONE unit of that schedule (a proposal or a
-//                  substep), each with exactly one cell lookup, so lanes that
-//                  cross a facet drift out of step with their neighbours
-//                  instead of stalling them, and a lane that finishes its
-//                  point takes the next point of its wave's range.  Per
-//                  point, the sequence of IEEE operations is the reference's.
+//                  while one lane does its ten substeps.  Here the lanes of
+//                  a wave step together while their points stay in their
+//                  cells and redo steps together when they have left them
+//                  (`advance`), and lanes that finish take the next points
+//                  of their wave's range.  Per point, the sequence of IEEE
+//                  operations is the reference's.
 //  * k_simple      calc_T_simple (calc_2Dto2D.cu:412-445).
 //  * k_velocity    calc_v (calc_2Dto2D.cu:561-602).
 //  * k_cell_idx    calc_cell_idx (calc_2Dto2D.cu:323-344).
@@ -278,128 +277,333 @@ __device__ __forceinline__ void stage_tables_prep(double* lds, const PrepSrc& ps
   __syncthreads();
 }
 
-// ----------------------------------------------------------------- trip
-// One unit of the reference's step schedule for one point (see k_integrate):
-//   k == 0: y = Trel_c [p;1]; if cell(y) == c accept, else start the RK2 redo
-//           (k = nStepsODE; p and c unchanged)   (calc_2Dto2D.cu:389-401)
-//   k >  0: one RK2 midpoint substep of A_c from p (solveODE, :179-194);
-//           p = y, c = cell(y), k--.
-// Both kinds of trip share the table read, the first affine product and the
-// cell lookup, so lanes in different modes diverge only over the midpoint
-// arithmetic.  (Measured on gfx950: evaluating the midpoint in every lane
-// and selecting, or chaining several Trel proposals speculatively so their
-// lookups overlap, are both slower than this.)
-// Returns true when the step is complete (the caller advances t).
-template <int DIM, int TESS, bool POW2, bool FAST = false, bool EARLY = true>
-__device__ __forceinline__ bool trip(double* p, int& c, int& k, const double*& row, int& nfb, const double* Ttab,
-                                     const double* Atab, double h, int nS, const Geom& g) {
-  constexpr int NE = DIM * (DIM + 1);
-  const bool fast = (k == 0);
-  double y[DIM];
-  affine<DIM>(y, row, p);
-  if (!fast) {  // RK2 midpoint substep (solveODE, calc_2Dto2D.cu:182-194)
-    // The reference's h * v / 2 is fl(h v) halved; (h / 2) * v rounds the
-    // same real number h v / 2, and halving commutes with rounding, so the
-    // two agree bit for bit unless |h v / 2| is subnormal (below 2^-1022).
-    // A nonzero v = A [p; 1] is at least ~2^-53 of its largest term, so that
-    // takes table entries near 1e-290.  One multiply per coordinate fewer.
-    const double hh = h * 0.5;
-    double m[DIM];
+// ---------------------------------------------------------- cell bounds
+// Lane masks (bits of inactive lanes are 0); uniform over the wave.
+__device__ __forceinline__ uint64_t lanes_lt(double a, double b) { return __builtin_amdgcn_fcmp(a, b, 4); }
+__device__ __forceinline__ uint64_t lanes_gt(double a, double b) { return __builtin_amdgcn_fcmp(a, b, 2); }
+__device__ __forceinline__ uint64_t lanes_ge(double a, double b) { return __builtin_amdgcn_fcmp(a, b, 3); }
+__device__ __forceinline__ uint64_t lanes_lt(int a, int b) { return __builtin_amdgcn_sicmp(a, b, 40); }
+__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
+// Whether points that came from their cells c are still in them, without a
+// lookup: a few affine functions of the point against bounds set once for the
+// cell.  The bounds lie g.eps inside the cell (the roundings of this test and
+// of the lookup's own arithmetic, and the lookup's clamp 1e-10 inside the far
+// walls), so a lane of inside(q) is one whose lookup of q gives c; one that is
+// turned down is looked up.  NaN and infinite points are turned down.
+//
+// Boxes (1D, type II): a lower and an upper bound per axis, none on the sides
+// of the domain (the lookup clamps, so what lies beyond belongs to the box).
+template <int DIM, int TESS>
+struct CellBounds {
+  double lo[DIM], hi[DIM];
+  __device__ __forceinline__ void enter(const double* p, int, const Geom& g) {
+    const int nC[3] = {g.nC0, g.nC1, g.nC2};
+    const double inc[3] = {g.inc_x, g.inc_y, g.inc_z}, rinc[3] = {g.rinc_x, g.rinc_y, g.rinc_z};
 #pragma unroll
-    for (int d = 0; d < DIM; d++) m[d] = p[d] + hh * y[d];
-    affine<DIM>(y, row, m);
+    for (int d = 0; d < DIM; d++) {
+      const double n1 = (double)(nC[d] - 1);
+      const double k = dmin(n1, dmax(0.0, __builtin_floor(p[d] * rinc[d])));
+      lo[d] = k > 0.0 ? (k + g.eps) * inc[d] : -__DBL_MAX__;
+      hi[d] = k < n1 ? (k + 1.0 - g.eps) * inc[d] : __DBL_MAX__;
+    }
+  }
+  __device__ __forceinline__ uint64_t inside(const double* q, const Geom&) const {
+    uint64_t in = ~0ull;
 #pragma unroll
-    for (int d = 0; d < DIM; d++) y[d] = p[d] + y[d] * h;
+    for (int d = 0; d < DIM; d++) in &= lanes_gt(q[d], lo[d]) & lanes_lt(q[d], hi[d]);
+    return in;
   }
-  const int cy = cell_of<DIM, TESS, POW2, FAST, EARLY>(y, g);
-  // (Measured on gfx950: the state update below written as selects instead
-  // of branches ran 3-4 % slower here and 11 % slower for 256 registration
-  // chains.)
-  if (!fast) {
+};
+
+// 2D triangles, s = p / inc: in triangle k of box (i, j) when u = sx - sy and
+// v = sx + sy lie on k's sides of i - j and i + j + 1 (the diagonals) and the
+// box edge is not crossed: sy is within the box for top and bottom, sx for
+// right and left.  A triangle on the domain's own side instead has the other
+// coordinate within the box: the lookup gives everything beyond that side
+// above (left of, ...) the box to it, and between the two diagonals the other
+// coordinate is within the box anyway.  Past a corner of the domain the
+// lookup's border is the diagonal's extension, so there the other coordinate
+// is bounded only to keep its rounding small (16 boxes out).
+template <>
+struct CellBounds<2, TESS_I> {
+  double k1, k2, ax, by, mid;
+  uint64_t above1, above2;  // lanes whose u lies at or above k1, whose v above k2
+  __device__ __forceinline__ void enter(const double* p, int c, const Geom& g) {
+    const double ni = (double)(g.nC0 - 1), nj = (double)(g.nC1 - 1);
+    const double i = dmin(ni, dmax(0.0, __builtin_floor(p[0] * g.rinc_x)));
+    const double j = dmin(nj, dmax(0.0, __builtin_floor(p[1] * g.rinc_y)));
+    // c & 3: 0 top, 1 right, 2 bottom, 3 left
+    const bool b1 = (c & 2) != 0;        // sx - i < sy - j
+    const bool b2 = ((c + 1) & 2) != 0;  // their sum > 1
+    above1 = ballot(!b1);
+    above2 = ballot(b2);
+    k1 = (i - j) + (b1 ? -g.eps : g.eps);
+    k2 = (i + j + 1.0) + (b2 ? g.eps : -g.eps);
+    const bool side = (c & 1) != 0;  // right, left
+    const double at = side ? i : j, last = side ? ni : nj;
+    const bool onwall = at == (b2 ? last : 0.0);  // (right and bottom look at the far wall)
+    const bool usex = side != onwall;
+    const double o = usex ? i : j, olast = usex ? ni : nj;
+    const double lo = onwall & (o == 0.0) ? -16.0 : o + g.eps;
+    const double hi = onwall & (o == olast) ? olast + 17.0 : o + 1.0 - g.eps;
+    // |w| < 1/2 for lo < s < hi
+    const double sc = 1.0 / (hi - lo);
+    ax = usex ? g.rinc_x * sc : 0.0;
+    by = usex ? 0.0 : g.rinc_y * sc;
+    mid = -0.5 * (lo + hi) * sc;
+  }
+  __device__ __forceinline__ uint64_t inside(const double* q, const Geom& g) const {
+    const double ty = q[1] * g.rinc_y;
+    const double u = __builtin_fma(q[0], g.rinc_x, -ty), v = __builtin_fma(q[0], g.rinc_x, ty);
+    const double w = __builtin_fma(q[0], ax, __builtin_fma(q[1], by, mid));
+    return ~((lanes_ge(u, k1) ^ above1) | (lanes_gt(v, k2) ^ above2)) & lanes_lt(__builtin_fabs(w), 0.5);
+  }
+};
+
+// 3D tetrahedra: in box (i, j, k) the four corner tetrahedra are cut off by
+// the planes sz -+ (sx + sy) and sz +- (sx - sy) at values that depend on the
+// box's orientation, and the central one lies on the inner side of all four.
+// A corner tetrahedron is bounded by one side of the box per axis besides.
+// At the domain's own walls those sides are moved out by half of g.eps (a
+// point kept on a wall by zero velocity is within rounding of it, either
+// side; the lookup clamps it, which moves each coordinate by at most g.eps,
+// hence four of them for the planes) -- but not the far z wall, past which
+// the lookup wraps or clamps z at another height (top_z uses inc_x).
+template <>
+struct CellBounds<3, TESS_I> {
+  double k1, k2, k3, k4, fx, fy, fz, zmax;
+  uint64_t a1, a2, a3, a4, lx, ly, lz;  // lanes above the planes, lanes whose side is the lower one
+  __device__ __forceinline__ void enter(const double* p, int c, const Geom& g) {
+    const double ni = (double)(g.nC0 - 1), nj = (double)(g.nC1 - 1), nk = (double)(g.nC2 - 1);
+    const double i = dmin(ni, dmax(0.0, __builtin_floor(p[0] * g.rinc_x)));
+    const double j = dmin(nj, dmax(0.0, __builtin_floor(p[1] * g.rinc_y)));
+    const double k = dmin(nk, dmax(0.0, __builtin_floor(p[2] * g.rinc_z)));
+    const int ii = (int)i, ij = (int)j, ik = (int)k;
+    // (another box than c's, next to a side, leaves 0 .. 4 and lies within no bounds)
+    const int tet = c - mul24(ii + mul24(ij, g.nC0) + mul24(ik, mul24(g.nC1, g.nC0)), 5);
+    const bool ok = (unsigned)tet < 5u;
+    const bool tf = ((ii + ij + ik) & 1) != 0;
+    const bool t1 = tet == 1, t2 = tet == 2, t3 = tet == 3, t4 = tet == 4;
+    const bool b1 = tf ? !t4 : t1, b2 = tf ? !t3 : t2, b3 = tf ? t1 : !t3, b4 = tf ? t2 : !t4;
+    const double e = 4.0 * g.eps;
+    k1 = (k - i - j - (tf ? 1.0 : 0.0)) + (b1 ? e : -e);
+    k2 = (k + i + j + (tf ? 1.0 : 2.0)) + (b2 ? e : -e);
+    k3 = (k + i - j + (tf ? 1.0 : 0.0)) + (b3 ? e : -e);
+    k4 = (k - i + j + (tf ? 1.0 : 0.0)) + (b4 ? e : -e);
+    a1 = ballot(b1);
+    a2 = ballot(b2);
+    a3 = ballot(b3);
+    a4 = ballot(b4);
+    const bool mid = tet == 0;  // no side
+    const bool ux = !mid & (tf ? t1 | t4 : t2 | t4), uy = !mid & (tf ? t2 | t4 : t2 | t3), uz = t1 | t2;
+    const double w = -0.5 * g.eps;  // a wall's bound is moved out
+    fx = mid ? -__DBL_MAX__ : (ux ? i + 1.0 - (i < ni ? e : w) : i + (i > 0.0 ? e : w)) * g.inc_x;
+    fy = mid ? -__DBL_MAX__ : (uy ? j + 1.0 - (j < nj ? e : w) : j + (j > 0.0 ? e : w)) * g.inc_y;
+    fz = mid ? -__DBL_MAX__ : (uz ? k + 1.0 - e : k + (k > 0.0 ? e : w)) * g.inc_z;
+    lx = ballot(!ux);
+    ly = ballot(!uy);
+    lz = ballot(!uz);
+    const double wall = dmin(((double)g.nC2 - e) * g.inc_z, g.top_z - e * g.inc_z);
+    zmax = ok ? wall : -__DBL_MAX__;
+  }
+  __device__ __forceinline__ uint64_t inside(const double* q, const Geom& g) const {
+    const double ty = q[1] * g.rinc_y;
+    const double s = __builtin_fma(q[0], g.rinc_x, ty), d = __builtin_fma(q[0], g.rinc_x, -ty);
+    const double d1 = __builtin_fma(q[2], g.rinc_z, -s), d2 = __builtin_fma(q[2], g.rinc_z, s);
+    const double d3 = __builtin_fma(q[2], g.rinc_z, d), d4 = __builtin_fma(q[2], g.rinc_z, -d);
+    return ~((lanes_gt(d1, k1) ^ a1) | (lanes_gt(d2, k2) ^ a2) | (lanes_gt(d3, k3) ^ a3) | (lanes_gt(d4, k4) ^ a4) |
+             (lanes_gt(q[0], fx) ^ lx) | (lanes_gt(q[1], fy) ^ ly) | (lanes_gt(q[2], fz) ^ lz)) &
+           lanes_lt(q[2], zmax) & lanes_lt(__builtin_fabs(d2), 0x1p30);
+  }
+};
+
+// -------------------------------------------------------------- advance
+// Integrates the calling lanes (t < tb on each) to step tb by the reference's
+// schedule (calc_2Dto2D.cu:385-402: every step the Trel proposal, and when it
+// leaves the cell nS RK2 substeps instead), in two phases taken in turn:
+//
+//   stretch  every lane whose point is in its cell by the bounds takes Trel
+//            steps, its row and bounds in registers, until its point leaves
+//            them or kSeg steps are done: nothing is looked up and no table
+//            is read, because the cell does not change.
+//   redo     the lanes that left look their proposal up: most left the cell
+//            and run the step's nS RK2 substeps, all of them together; some
+//            were only beside a facet and accept it.
+//
+// Per point the sequence of IEEE operations is the reference's.
+//
+// What bounds calc_T is instruction issue: a wave alone on its SIMD issues an
+// FP64 operation every 8 cycles, dependent or not, several waves one every 4;
+// a launch of few waves ends with its slowest one.  A step of a stretch is 24
+// VALU and 9 scalar instructions (2D type I: 8 the affine product, 8 the
+// bounds, 8 the update) against 36 and 20 and LDS latency for a trip in
+// lockstep (one unit, proposal or substep, of every lane, its cell looked up
+// and its row read each time; see `trip`), or 52 when some lane of the wave
+// is at a redone step.  The loop has no divergent branch: lanes that have
+// left stay where they are by selects.  A redo costs about as much as 20
+// steps of a stretch however many lanes share it, and a lane that waits for
+// company delays the wave's end: hence kSeg (16, 24, 32 and 100 steps: 2D
+// 2 000 000 points 534, 470, 448 us; 3D volume warp 351, 319, 308, 341 us).
+// On MI355X, lockstep -> this: 2D random points, 1 000: 51 -> 41 us, 65 536:
+// 56 -> 45, 2 000 000: 606 -> 430; grids, 512 x 512: 67 -> 67 (its slowest
+// waves cross many facets), 2048 x 2048: 735 -> 580; 640 x 480 with fields
+// that leave the image 175 -> 137; 1D, 10^6 points of 50 cells 274 -> 195;
+// 3D, 64 x 80 x 96 volume 331 -> 308.
+//
+// more: the caller has further points for lanes that finish; then it returns
+// as soon as `refill` lanes have.
+constexpr int kSeg = 32;
+constexpr int kSegTraj = 12;  // calc_trajectory: lanes far apart in steps store to as many rows (16: +3 %, 8: +6 %)
+constexpr int kRefill = 8;
+
+// The point at the domain's corner (0, 0).  With zero velocity on the walls
+// its velocity is zero up to rounding: it drifts ~1e-16 out of the domain and
+// with some fields flips between triangles 0 and 3 of box (0, 0) at every
+// substep, so up to all its steps are redone, one dependent chain of 1 100
+// units where its neighbours have ~110, and the wave (a launch of 512 x 512
+// grid points: all of it) waits for it.  Alone in its wave it runs here to
+// step tb: the two triangles' rows stay in registers, a branch picks one, and
+// the lookup is two products and three comparisons while the point is within
+// an eighth of a box of the corner, where the reference's rules
+// (calc_2Dto2D.cu:60-110) come down to: left of the corner (px <= 0) triangle
+// 3 unless sy < sx, else 3 where sx < sy and 0 elsewhere (1 - x < y holds for
+// no point this near).  Returns where it has left that neighbourhood.
+template <int MODE>
+__device__ __forceinline__ void corner_steps(double* p, int& c, int& t, int tb, int& nfb, const double* Ttab,
+                                             const double* Atab, double h, int nS, const Geom& g,
+                                             double* __restrict__ traj, int64_t nPts) {
+  const double hh = h * 0.5, mx = 0.125 * g.inc_x, my = 0.125 * g.inc_y;
+  double A0[6], A3[6];
 #pragma unroll
-    for (int d = 0; d < DIM; d++) p[d] = y[d];
-    const bool done = --k == 0;
-    row = (done ? Ttab : Atab) + mul24(cy, NE);  // (the same row when the cell did not change)
-    c = cy;
-    return done;
+  for (int e = 0; e < 6; e++) {
+    A0[e] = Atab[e];
+    A3[e] = Atab[18 + e];
   }
-  if (cy == c) {
-#pragma unroll
-    for (int d = 0; d < DIM; d++) p[d] = y[d];
-    return true;
+  // The cell of q, wave-uniform as there is one lane (its branches are then
+  // scalar ones); `near` false: looked up, the point is not beside the corner.
+  auto cell = [&](const double* q, bool& near) {
+    near = (lanes_lt(__builtin_fabs(q[0]), mx) & lanes_lt(__builtin_fabs(q[1]), my)) != 0;
+    if (!near) return (int)__builtin_amdgcn_readfirstlane(cell2<TESS_I, true>(q, g));
+    const double sx = q[0] * g.rinc_x, sy = q[1] * g.rinc_y;
+    const uint64_t left = lanes_lt(sx, sy) | (~lanes_gt(q[0], 0.0) & ~lanes_lt(sy, sx) & __builtin_amdgcn_read_exec());
+    return left != 0 ? 3 : 0;
+  };
+  auto substep = [&](const double* A) {
+    double y[2], m[2];
+    affine<2>(y, A, p);
+    m[0] = p[0] + hh * y[0];
+    m[1] = p[1] + hh * y[1];
+    affine<2>(y, A, m);
+    p[0] = p[0] + y[0] * h;
+    p[1] = p[1] + y[1] * h;
+  };
+  bool near = true;
+  int cu = __builtin_amdgcn_readfirstlane(c);
+  const int te = __builtin_amdgcn_readfirstlane(tb);
+  int tu = __builtin_amdgcn_readfirstlane(t);
+  while (near && tu < te) {
+    double y[2];
+    affine<2>(y, Ttab + cu * 6, p);
+    const int cy = cell(y, near);
+    if (cy == cu) {
+      p[0] = y[0];
+      p[1] = y[1];
+    } else {
+      nfb++;
+      for (int s = 0; s < nS; s++) {
+        if (cu == 0) substep(A0);
+        else if (cu == 3) substep(A3);
+        else substep(Atab + cu * 6);
+        cu = cell(p, near);
+      }
+    }
+    if (MODE == 1) store_pt<2>(traj, (int64_t)tu * nPts, p);
+    tu++;
   }
-  nfb++;
-  if (nS > 0) {
-    k = nS;
-    row = Atab + mul24(c, NE);
-    return false;
-  }
-  return true;  // zero substeps: the step leaves p where it was
+  c = cu;
+  t = tu;
 }
 
-// ------------------------------------------------------------ lone lane
-// A wave left with a single unfinished lane runs one dependent chain of
-// instructions, so its trips cost their latency (a dependent FP64 operation
-// takes 16-22 cycles on MI355X), not their issue.  The point that gets there
-// is the domain corner (0, 0): its velocity is zero up to rounding, it
-// drifts just outside the domain, and the Trel proposal leaves the cell at
-// most steps, so the lane runs up to 1 100 trips while its neighbours need
-// ~104.  (In the registration step, where only its FP32 sample matters, a
-// bound on its path usually fixes that sample and the pixel is left out:
-// corner_sample_is_src00.)  Here the lane loops on its own: its branches are
-// uniform (one lane), each trip does only its own kind of work, and the lookup is branch-free
-// (cell2_flat, no strict-interior test).  Measured on the one-chain
-// registration: ~770 instead of ~940 cycles a trip, +5 % at 40 slots, +11 %
-// at 24.  (Holding the table row in registers took the step kernel past 64
-// VGPRs; reading the row with scalar loads from a global copy of the tables,
-// the cell being wave-uniform here, measured 1-2 % slower than LDS.)  Same
-// schedule and IEEE operations as `trip`.  Runs until t >= tb and leaves row
-// consistent with (c, k).
-template <int DIM, int TESS, bool POW2>
-__device__ __forceinline__ int lone_cell(const double* y, const Geom& g) {
-  if (DIM == 2 && TESS == TESS_I && POW2) return cell2_flat(y, g);
-  return cell_of<DIM, TESS, POW2>(y, g);
-}
-
-template <int DIM, int TESS, bool POW2>
-__device__ __forceinline__ void lone_trips(double* p, int& c, int& k, int& t, int tb, const double*& row, int& nfb,
-                                           const double* Ttab, const double* Atab, double h, int nS,
-                                           const Geom& g) {
+template <int DIM, int TESS, bool POW2, int MODE>
+__device__ __forceinline__ void advance(double* p, int& c, int& t, int tb, int& nfb, const double* Ttab,
+                                        const double* Atab, double h, int nS, const Geom& g, bool more_,
+                                        int refill, double* __restrict__ traj, int64_t nPts) {
   constexpr int NE = DIM * (DIM + 1);
-  const double hh = h * 0.5;  // as in `trip`
-  while (t < tb) {
-    const double* r = row;
-    double y[DIM];
-    affine<DIM>(y, r, p);
-    if (k == 0) {  // Trel proposal
-      const int cy = lone_cell<DIM, TESS, POW2>(y, g);
+  // The reference's h * v / 2 is fl(h v) halved; (h / 2) * v rounds the same
+  // real number h v / 2, and halving commutes with rounding, so the two agree
+  // bit for bit unless |h v / 2| is subnormal (below 2^-1022).  A nonzero
+  // v = A [p; 1] is at least ~2^-53 of its largest term, so that takes table
+  // entries near 1e-290.  One multiply per coordinate fewer.
+  const double hh = h * 0.5;
+  const int nAll = __popcll(__builtin_amdgcn_read_exec());
+  constexpr int seg = MODE == 1 ? kSegTraj : kSeg;
+  const bool more = __builtin_amdgcn_readfirstlane((int)more_) != 0;  // (wave-uniform: kept in scalar registers)
+  int cool = 0;  // rounds without a stretch (wave-uniform)
+  for (;;) {
+    const uint64_t todo = ballot(t < tb);
+    const int nTodo = __popcll(todo);
+    if (nTodo == 0 || (more && nAll - nTodo >= refill)) break;
+    bool waits = t < tb;  // the lane takes part in the redo phase
+    if (DIM == 2 && TESS == TESS_I && POW2 && nTodo == 1 && cool > 0) {  // one lane left, and no stretch for it
+      if (waits && (c == 0 || c == 3) && __builtin_fabs(p[0]) < 0.125 * g.inc_x &&
+          __builtin_fabs(p[1]) < 0.125 * g.inc_y) {
+        corner_steps<MODE>(p, c, t, tb, nfb, Ttab, Atab, h, nS, g, traj, nPts);
+        waits = false;
+      }
+    }
+    if (cool > 0) {
+      cool--;
+    } else {
+      CellBounds<DIM, TESS> B;
+      double R[NE];
+      const double* row = Ttab + mul24(c, NE);
+#pragma unroll
+      for (int e = 0; e < NE; e++) R[e] = row[e];
+      B.enter(p, c, g);
+      uint64_t go = B.inside(p, g) & todo;  // the lanes of the stretch
+      if (go == 0) cool = 8;
+      for (;;) {
+        const int lim = tb - t < seg ? tb : t + seg;
+        while (go != 0) {
+          double y[DIM];
+          affine<DIM>(y, R, p);
+          go &= B.inside(y, g) & lanes_lt(t, lim);
+          const bool in = lane_in(go);
+#pragma unroll
+          for (int d = 0; d < DIM; d++) p[d] = in ? y[d] : p[d];
+          if (MODE == 1 && in) store_pt<DIM>(traj, (int64_t)t * nPts, p);
+          t += in ? 1 : 0;
+        }
+        waits = t < lim;
+        go = ballot(t < tb);  // with no lane waiting the cells are still the same
+        if (go == 0 || ballot(waits) != 0 || (more && nAll - __popcll(go) >= refill)) break;
+      }
+    }
+    if (waits) {
+      const double* row = Ttab + mul24(c, NE);
+      double y[DIM];
+      affine<DIM>(y, row, p);
+      const int cy = cell_of<DIM, TESS, POW2, true>(y, g);
       if (cy == c) {
 #pragma unroll
         for (int d = 0; d < DIM; d++) p[d] = y[d];
-        t++;
       } else {
         nfb++;
-        if (nS > 0) {
-          k = nS;
+        for (int s = 0; s < nS; s++) {
           row = Atab + mul24(c, NE);
-        } else {
-          t++;
+          affine<DIM>(y, row, p);
+          double m[DIM];
+#pragma unroll
+          for (int d = 0; d < DIM; d++) m[d] = p[d] + hh * y[d];
+          affine<DIM>(y, row, m);
+#pragma unroll
+          for (int d = 0; d < DIM; d++) p[d] = p[d] + y[d] * h;
+          c = cell_of<DIM, TESS, POW2, true>(p, g);
         }
       }
-    } else {  // one RK2 midpoint substep
-      double m[DIM];
-#pragma unroll
-      for (int d = 0; d < DIM; d++) m[d] = p[d] + hh * y[d];
-      affine<DIM>(y, r, m);
-#pragma unroll
-      for (int d = 0; d < DIM; d++) y[d] = p[d] + y[d] * h;
-      const int cy = lone_cell<DIM, TESS, POW2>(y, g);
-#pragma unroll
-      for (int d = 0; d < DIM; d++) p[d] = y[d];
-      const bool done = --k == 0;
-      if (done | (cy != c)) row = (done ? Ttab : Atab) + mul24(cy, NE);
-      c = cy;
-      if (done) t++;
+      if (MODE == 1) store_pt<DIM>(traj, (int64_t)t * nPts, p);
+      t++;
     }
   }
 }
@@ -408,15 +612,11 @@ __device__ __forceinline__ void lone_trips(double* p, int& c, int& k, int& t, in
 // MODE 0: calc_T (write the end point).  MODE 1: calc_trajectory (write the
 // point after every step into traj[(t*nPts + i)*DIM]).
 //
-// Lane state: p (current point), c (cell of p), t (steps done),
-// k (RK2 substeps still to run for the current step; 0 = next trip is a
-// Trel proposal); one loop trip is one `trip`.  solveODE recomputes cell(p)
-// at the top of every substep; here it is the lookup at the end of the
-// previous trip, of the same p: same value.
+// Lane state: p (current point), c (cell of p), t (steps done).  solveODE
+// recomputes cell(p) at the top of every substep; here it is the lookup at
+// the end of the previous one, of the same p: same value.  Lanes retire and
+// take the next points of the wave's range between calls of `advance`.
 //
-// Trips run in an inner loop until some lane finishes its point; only then
-// do lanes retire and refill from the wave's range (the bookkeeping costs
-// ballots and branches, so it stays out of the per-trip path).
 // Processing index i -> point index when the points form a row-major grid
 // of row length w (a multiple of 8): the first nTiled = 8 w floor(nPts / 8 w)
 // indices walk 8 x 8 tiles (64 consecutive indices one tile, the tiles of
@@ -435,18 +635,21 @@ __device__ __forceinline__ int64_t tile_order(int64_t i, int w, int64_t nTiled) 
 // (indices into pos0, out and nfb_out; with gw > 0 through tile_order, with
 // lord through lbase + lord[i - lbase], a tile's order held in LDS).
 // Wave-uniform arguments; every lane of the wave calls it.
-template <int DIM, int TESS, bool POW2, int MODE, bool FAST = false>
+template <int DIM, int TESS, bool POW2, int MODE>
 __device__ __forceinline__ void integrate_range(int64_t begin, int64_t end, const double* __restrict__ pos0,
                                                 double* __restrict__ out, const double* Ttab, const double* Atab,
                                                 double h, int nT, int nS, int64_t nPts, const Geom& g,
                                                 int32_t* __restrict__ nfb_out, int gw = 0,
                                                 const uint16_t* lord = nullptr, int64_t lbase = 0) {
   const int64_t nTiled = gw > 0 ? nPts / (8 * (int64_t)gw) * (8 * (int64_t)gw) : 0;
-  constexpr int NE = DIM * (DIM + 1);
+  // a grid's tiles are 64 neighbouring points that need similar work, so a
+  // wave takes one after another (2048 x 2048 points: 750 -> 610 us); other
+  // waves take the next points as soon as kRefill lanes are free (256 batched
+  // instances, 8 instead of 16: 14.3 -> 13.9 ms, 32: 16.7; 64: 15.3)
+  const int refill = gw > 0 ? 64 : kRefill;
   int64_t next = begin;  // wave-uniform cursor into [begin, end)
   double p[DIM];
-  int c = 0, t = 0, k = 0, nfb = 0;
-  const double* row = Ttab;  // the table row the next trip reads
+  int c = 0, t = 0, nfb = 0;
   int64_t my = 0;
   bool active = false;
   for (;;) {
@@ -464,9 +667,7 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int64_t end, cons
           active = true;
           load_pt<DIM>(pos0, my, p);
           c = cell_of<DIM, TESS, POW2>(p, g);
-          row = Ttab + mul24(c, NE);
           t = 0;
-          k = 0;
           nfb = 0;
         }
       }
@@ -474,31 +675,13 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int64_t end, cons
     }
     if (ballot(active) == 0) break;
     if (!active || t >= nT) continue;
-    if (MODE == 0 && DIM == 2 && __popcll(__builtin_amdgcn_read_exec()) == 1) {  // one lane left: its own loop
-      lone_trips<DIM, TESS, POW2>(p, c, k, t, nT, row, nfb, Ttab, Atab, h, nS, g);
-      continue;
-    }
-    // Trips until some lane of the region finishes its point, two per loop
-    // iteration with the exit test between them (written out: the compiler
-    // does not unroll a loop around a ballot), so the point's registers
-    // alternate instead of being copied back at the end of every trip.
-    for (;;) {
-      if (trip<DIM, TESS, POW2, FAST>(p, c, k, row, nfb, Ttab, Atab, h, nS, g)) {
-        if (MODE == 1) store_pt<DIM>(out, (int64_t)t * nPts + my, p);
-        t++;
-      }
-      if (ballot(t >= nT) != 0) break;
-      if (trip<DIM, TESS, POW2, FAST>(p, c, k, row, nfb, Ttab, Atab, h, nS, g)) {
-        if (MODE == 1) store_pt<DIM>(out, (int64_t)t * nPts + my, p);
-        t++;
-      }
-      if (ballot(t >= nT) != 0) break;
-    }
+    advance<DIM, TESS, POW2, MODE>(p, c, t, nT, nfb, Ttab, Atab, h, nS, g, next < end, refill,
+                                   MODE == 1 ? out + my * DIM : nullptr, nPts);
   }
 }
 
-template <int DIM, int TESS, bool POW2, bool LDS, int MODE, bool FAST = false>
-__global__ void __launch_bounds__(1024)
+template <int DIM, int TESS, bool POW2, bool LDS, int MODE>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5)))
     k_integrate(const double* __restrict__ pos0, double* __restrict__ out,
                 const double* __restrict__ Trels, const double* __restrict__ As, double h,
                 int nT, int nS, int64_t nPts, Geom g, int nC, int ptsPerWave,
@@ -509,7 +692,7 @@ __global__ void __launch_bounds__(1024)
   // length W (the first index, a multiple of 8 up to 8 x blockDim.x, where y
   // changes from point 0's), so that waves take 8 x 8 tiles: neighbouring
   // points flow alike and cross facets at about the same steps, so a wave's
-  // lanes need similar numbers of trips.  Only the processing order depends
+  // lanes need similar numbers of steps.  Only the processing order depends
   // on it (every point's result is its own), so a wrong guess costs time
   // only.  The loads are issued before the tables are staged.
   __shared__ int grid_w;
@@ -543,7 +726,7 @@ __global__ void __launch_bounds__(1024)
   const int64_t begin = wave * (int64_t)ptsPerWave;
   if (begin >= nPts) return;
   const int64_t end = begin + ptsPerWave < nPts ? begin + ptsPerWave : nPts;
-  integrate_range<DIM, TESS, POW2, MODE, FAST>(begin, end, pos0, out, Ttab, Atab, h, nT, nS, nPts, g, nfb_out, gw);
+  integrate_range<DIM, TESS, POW2, MODE>(begin, end, pos0, out, Ttab, Atab, h, nT, nS, nPts, g, nfb_out, gw);
 }
 
 // ---------------------------------------------------------- sensitivity

@@ -47,6 +47,136 @@
 
 namespace cpab {
 
+// ----------------------------------------------------------------- trip
+// The registration step integrates in lockstep (calc_T's two phases, `advance`,
+// measured 6 % slower here: 79 instead of 63 VGPRs leave fewer waves, and a
+// wave that ends later tells later slots later that they are not needed).
+// One unit of the reference's step schedule for one point of a lane (all lanes of a wave in lockstep, whatever unit each is at):
+//   k == 0: y = Trel_c [p;1]; if cell(y) == c accept, else start the RK2 redo
+//           (k = nStepsODE; p and c unchanged)   (calc_2Dto2D.cu:389-401)
+//   k >  0: one RK2 midpoint substep of A_c from p (solveODE, :179-194);
+//           p = y, c = cell(y), k--.
+// Both kinds of trip share the table read, the first affine product and the
+// cell lookup, so lanes in different modes diverge only over the midpoint
+// arithmetic.  (Measured on gfx950: evaluating the midpoint in every lane
+// and selecting, or chaining several Trel proposals speculatively so their
+// lookups overlap, are both slower than this.)
+// Returns true when the step is complete (the caller advances t).
+template <int DIM, int TESS, bool POW2, bool FAST = false, bool EARLY = true>
+__device__ __forceinline__ bool trip(double* p, int& c, int& k, const double*& row, int& nfb, const double* Ttab,
+                                     const double* Atab, double h, int nS, const Geom& g) {
+  constexpr int NE = DIM * (DIM + 1);
+  const bool fast = (k == 0);
+  double y[DIM];
+  affine<DIM>(y, row, p);
+  if (!fast) {  // RK2 midpoint substep (solveODE, calc_2Dto2D.cu:182-194)
+    // The reference's h * v / 2 is fl(h v) halved; (h / 2) * v rounds the
+    // same real number h v / 2, and halving commutes with rounding, so the
+    // two agree bit for bit unless |h v / 2| is subnormal (below 2^-1022).
+    // A nonzero v = A [p; 1] is at least ~2^-53 of its largest term, so that
+    // takes table entries near 1e-290.  One multiply per coordinate fewer.
+    const double hh = h * 0.5;
+    double m[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; d++) m[d] = p[d] + hh * y[d];
+    affine<DIM>(y, row, m);
+#pragma unroll
+    for (int d = 0; d < DIM; d++) y[d] = p[d] + y[d] * h;
+  }
+  const int cy = cell_of<DIM, TESS, POW2, FAST, EARLY>(y, g);
+  // (Measured on gfx950: the state update below written as selects instead
+  // of branches ran 3-4 % slower here and 11 % slower for 256 registration
+  // chains.)
+  if (!fast) {
+#pragma unroll
+    for (int d = 0; d < DIM; d++) p[d] = y[d];
+    const bool done = --k == 0;
+    row = (done ? Ttab : Atab) + mul24(cy, NE);  // (the same row when the cell did not change)
+    c = cy;
+    return done;
+  }
+  if (cy == c) {
+#pragma unroll
+    for (int d = 0; d < DIM; d++) p[d] = y[d];
+    return true;
+  }
+  nfb++;
+  if (nS > 0) {
+    k = nS;
+    row = Atab + mul24(c, NE);
+    return false;
+  }
+  return true;  // zero substeps: the step leaves p where it was
+}
+
+// ------------------------------------------------------------ lone lane
+// A wave left with a single unfinished lane runs one dependent chain of
+// instructions, so its trips cost their latency (a dependent FP64 operation
+// takes 16-22 cycles on MI355X), not their issue.  The point that gets there
+// is the domain corner (0, 0): its velocity is zero up to rounding, it
+// drifts just outside the domain, and the Trel proposal leaves the cell at
+// most steps, so the lane runs up to 1 100 trips while its neighbours need
+// ~104.  (In the registration step, where only its FP32 sample matters, a
+// bound on its path usually fixes that sample and the pixel is left out:
+// corner_sample_is_src00.)  Here the lane loops on its own: its branches are
+// uniform (one lane), each trip does only its own kind of work, and the lookup is branch-free
+// (cell2_flat, no strict-interior test).  Measured on the one-chain
+// registration: ~770 instead of ~940 cycles a trip, +5 % at 40 slots, +11 %
+// at 24.  (Holding the table row in registers took the step kernel past 64
+// VGPRs; reading the row with scalar loads from a global copy of the tables,
+// the cell being wave-uniform here, measured 1-2 % slower than LDS.)  Same
+// schedule and IEEE operations as `trip`.  Runs until t >= tb and leaves row
+// consistent with (c, k).
+template <int DIM, int TESS, bool POW2>
+__device__ __forceinline__ int lone_cell(const double* y, const Geom& g) {
+  if (DIM == 2 && TESS == TESS_I && POW2) return cell2_flat(y, g);
+  return cell_of<DIM, TESS, POW2>(y, g);
+}
+
+template <int DIM, int TESS, bool POW2>
+__device__ __forceinline__ void lone_trips(double* p, int& c, int& k, int& t, int tb, const double*& row, int& nfb,
+                                           const double* Ttab, const double* Atab, double h, int nS,
+                                           const Geom& g) {
+  constexpr int NE = DIM * (DIM + 1);
+  const double hh = h * 0.5;  // as in `trip`
+  while (t < tb) {
+    const double* r = row;
+    double y[DIM];
+    affine<DIM>(y, r, p);
+    if (k == 0) {  // Trel proposal
+      const int cy = lone_cell<DIM, TESS, POW2>(y, g);
+      if (cy == c) {
+#pragma unroll
+        for (int d = 0; d < DIM; d++) p[d] = y[d];
+        t++;
+      } else {
+        nfb++;
+        if (nS > 0) {
+          k = nS;
+          row = Atab + mul24(c, NE);
+        } else {
+          t++;
+        }
+      }
+    } else {  // one RK2 midpoint substep
+      double m[DIM];
+#pragma unroll
+      for (int d = 0; d < DIM; d++) m[d] = p[d] + hh * y[d];
+      affine<DIM>(y, r, m);
+#pragma unroll
+      for (int d = 0; d < DIM; d++) y[d] = p[d] + y[d] * h;
+      const int cy = lone_cell<DIM, TESS, POW2>(y, g);
+#pragma unroll
+      for (int d = 0; d < DIM; d++) p[d] = y[d];
+      const bool done = --k == 0;
+      if (done | (cy != c)) row = (done ? Ttab : Atab) + mul24(cy, NE);
+      c = cy;
+      if (done) t++;
+    }
+  }
+}
+
+
 struct Philox {
   uint32_t x0, x1, x2, x3;
 };
@@ -722,7 +852,7 @@ __global__ void __launch_bounds__(BLOCK) k_mcmc_step(McmcDesc D, int init) {
           lone_trips<2, TESS, POW2>(p, c, k, t, tb, row, nfb, Ttab, Atab, h, nS, g);
           continue;
         }
-        for (;;) {  // two trips per iteration, as in integrate_range
+        for (;;) {  // two trips per iteration (written out: the compiler does not unroll around a ballot)
           if (trip<2, TESS, POW2, FAST, !SWAP>(p, c, k, row, nfb, Ttab, Atab, h, nS, g)) t++;
           if (ballot(t >= tb) != 0) break;
           if (trip<2, TESS, POW2, FAST, !SWAP>(p, c, k, row, nfb, Ttab, Atab, h, nS, g)) t++;
