@@ -553,8 +553,14 @@ int cpab_calc_v(cpab_ctx* ctx, int dim, int tess, int nC, const double* pts, dou
   if (overlap(pts, pb, vel, pb)) return fail(ctx, CPAB_ERR_ALIAS, "pts and v cannot point to the same memory");
   const size_t tb = (size_t)nC * dim * (dim + 1) * sizeof(double);
   const bool lds = tb <= (size_t)ctx->max_lds;
-  const int block = 256;
-  const dim3 grid((unsigned)((nPts + block - 1) / block));
+  // blocks that walk over the points, as many as the chip holds at once (a
+  // large table leaves room for few, so those are larger: 48 KiB, three of
+  // 512 threads a CU)
+  const int block = tb > 16384 ? 512 : 256;
+  int per_cu = 2048 / block;
+  if (lds && tb > 0 && per_cu > (int)((size_t)ctx->max_lds / tb)) per_cu = (int)((size_t)ctx->max_lds / tb);
+  const int64_t all = (nPts + block - 1) / block, most = (int64_t)ctx->n_cu * per_cu;
+  const dim3 grid((unsigned)(all < most ? all : most));
   DISPATCH_GEOM(dim, tess, pow2, {
     if (lds) {
       auto k = k_velocity<D_, T_, P_, true>;

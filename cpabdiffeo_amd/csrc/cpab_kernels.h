@@ -834,6 +834,11 @@ __global__ void __launch_bounds__(1024)
   store_pt<DIM>(out, i, p);
 }
 
+// calc_v: bound by memory (one point read, one velocity written).  A block
+// stages the table once and walks over the points; a block per 256 points
+// staged a table of 1 024 cells (48 KiB) for 8 KiB of points.  On MI355X,
+// 2048 x 2048 points: 1 024 cells 90.5 -> 24.1 us (5.6 TB/s), 64 cells 21.5 ->
+// 21.7 us; two or four points loaded ahead in each thread measured the same.
 template <int DIM, int TESS, bool POW2, bool LDS>
 __global__ void __launch_bounds__(1024)
     k_velocity(const double* __restrict__ pts, double* __restrict__ vel, const double* __restrict__ As,
@@ -846,12 +851,13 @@ __global__ void __launch_bounds__(1024)
     __syncthreads();
     Atab = lds;
   }
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nPts) return;
-  double p[DIM], v[DIM];
-  load_pt<DIM>(pts, i, p);
-  affine<DIM>(v, Atab + cell_of<DIM, TESS, POW2>(p, g) * NE, p);
-  store_pt<DIM>(vel, i, v);
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nPts; i += stride) {
+    double p[DIM], v[DIM];
+    load_pt<DIM>(pts, i, p);
+    affine<DIM>(v, Atab + cell_of<DIM, TESS, POW2>(p, g) * NE, p);
+    store_pt<DIM>(vel, i, v);
+  }
 }
 
 template <int DIM, int TESS, bool POW2>
