@@ -173,14 +173,16 @@ class Calcs:
         return grad_per_point
 
     def calc_trajectory(self, xmins, xmaxs, Tlocals_vectorized, As_vectorized, pts0, dt, nTimeSteps,
-                        nStepsOdeSolver, dim_domain, dim_range, nCs, incs):
+                        nStepsOdeSolver, dim_domain, dim_range, nCs, incs, out=None):
         """cpab/gpu/Calcs.py:735-814.  Returns a device tensor (nTimeSteps, nPts, dim):
-        row t is the position after t+1 steps."""
+        row t is the position after t+1 steps (written into `out` when given)."""
         dim = dim_domain
         T, A = self._tables(dim, Tlocals_vectorized, As_vectorized)
         p0 = self._pts(pts0, dim)
         torch = torch_mod()
-        traj = torch.empty((int(nTimeSteps), p0.shape[0], dim), dtype=torch.float64, device=p0.device)
+        shape = (int(nTimeSteps), p0.shape[0], dim)
+        traj = (torch.empty(shape, dtype=torch.float64, device=p0.device) if out is None
+                else dev_tensor(out, "float64", shape))
         ctx = context_for(p0)
         ctx.call("cpab_calc_trajectory", dim, self.tess_type, self.nCells, p0.data_ptr(),
                  traj.data_ptr(), T.data_ptr(), A.data_ptr(), float(dt), int(nTimeSteps),

@@ -474,10 +474,13 @@ class CpaSpace:
         nT = int(params_flow_int["nTimeSteps"])
         nS = params_flow_int.get("nStepsODEsolver", 100)
         sA, T = self.prepare_signed_As_and_Tlocals(mysign, dt, pat)
-        traj = self._gpu_calcs.calc_trajectory(None, None, T, sA, pts, dt, nT, nS, self.dim_domain,
-                                               self.dim_range, self.nCs, self.incs)
+        # one buffer, its first row pts: the rows after it are written in place
         p0 = dev_tensor(pts, "float64")
-        return CpuGpuArray.from_gpu(torch.cat([p0[None], traj], dim=0))
+        traj = torch.empty((1 + nT,) + tuple(p0.shape), dtype=torch.float64, device=p0.device)
+        traj[0].copy_(p0)
+        self._gpu_calcs.calc_trajectory(None, None, T, sA, pts, dt, nT, nS, self.dim_domain, self.dim_range,
+                                        self.nCs, self.incs, out=traj[1:])
+        return CpuGpuArray.from_gpu(traj)
 
     def __repr__(self):
         return "CpaSpace(dim=%d, tess=%s, nCs=%s, nC=%d, d=%d)" % (
