@@ -3,6 +3,7 @@
 // include/cpab_hip.h.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -857,6 +858,10 @@ int batch_tiles(cpab_batch* b, int tile) {
     }
   }
   if (t.size() > 0x7fffffff) return fail(ctx, CPAB_ERR_ARG, "too many tiles");
+  // the largest first (a tile of 16 384 points is over a millisecond of a
+  // CU), so the instances' remainders even out the end of the launch
+  std::stable_sort(t.begin(), t.end(),
+                   [](const BatchTile& x, const BatchTile& y) { return x.end - x.begin > y.end - y.begin; });
   HIP_OK(ctx, hipStreamSynchronize(ctx->stream));
   if (b->d_tiles) HIP_OK(ctx, hipFree(b->d_tiles));
   b->d_tiles = nullptr;

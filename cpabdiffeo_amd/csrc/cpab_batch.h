@@ -3,12 +3,12 @@
 // Each instance has its own tessellation (cell counts, increments), its own
 // tables (Trels then signed As, staged per instance in one table buffer) and
 // its own point range in one concatenated point buffer.  The host cuts every
-// instance into tiles of at most `tile` points (in instance order) and the
-// kernel's blocks take `chunk` consecutive tiles at a time from a queue (one
-// atomic per chunk; a block leaves when the queue is exhausted, so every
+// instance into tiles of at most `tile` points (the largest first) and the
+// kernel's blocks take up to `chunk` consecutive tiles at a time from a queue
+// (one atomic per grab; a block leaves when the queue is exhausted, so every
 // block ends).  A block keeps the tables of the instance it is working on in
 // LDS and reloads them only when a tile of another instance comes; the waves
-// of a block split the tile's points and integrate them with
+// of a block draw the tile's points from one cursor and integrate them with
 // k_integrate's two phases (`advance`).  Per point the arithmetic is exactly calc_T's, so a
 // point gives the same bits batched or alone.
 #pragma once
@@ -75,6 +75,7 @@ __global__ void k_batch_reset(unsigned int* queue) {
 // when, never the point's result.
 constexpr int kBucketTileMax = 16384;  // the most points of a sorted tile (16-bit indices)
 constexpr int kBucketMax = 1024;       // buckets
+constexpr int kItemMax = 1 << 30;      // the most points of an item taken at a time (32-bit cursor)
 
 template <int DIM>
 __device__ __forceinline__ int bucket_of(const double* p, const double* sc, int nb) {
@@ -142,20 +143,30 @@ __global__ void __launch_bounds__(1024)
                       int32_t* __restrict__ nfb_out, int sort_off) {
   constexpr int NE = DIM * (DIM + 1);
   extern __shared__ double lds[];
-  __shared__ int s_t0;
+  __shared__ int s_t0, s_t1, cursor;
   // sort_off > 0: the tiles' processing order by position, in LDS after
   // the tables (sort_off doubles in): bucket counters, then indices
   unsigned int* hist = reinterpret_cast<unsigned int*>(lds + sort_off);
   uint16_t* idx = reinterpret_cast<uint16_t*>(hist + kBucketMax);
-  const int nw = blockDim.x >> 6, w = threadIdx.x >> 6;
   int cur = -1;  // instance whose tables are in LDS (block-uniform)
   for (;;) {
     __syncthreads();  // every wave is done with the previous chunk's s_t0
-    if (threadIdx.x == 0) s_t0 = (int)atomicAdd(queue, (unsigned int)chunk);
+    if (threadIdx.x == 0) {
+      // `chunk` tiles at a time while each block has four such grabs ahead of
+      // it, then fewer, in the end one (256 instances, tiles of 16 384, chunk
+      // 4: 2 400 tiles are 2.3 grabs for each of 256 blocks, and the launch
+      // waited for those that took three)
+      const unsigned int seen = __hip_atomic_load(queue, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int left = seen < (unsigned int)nTiles ? nTiles - (int)seen : 0;
+      int k = left / (4 * (int)gridDim.x);
+      k = k < 1 ? 1 : (k > chunk ? chunk : k);
+      s_t0 = (int)atomicAdd(queue, (unsigned int)k);
+      s_t1 = s_t0 + k;
+    }
     __syncthreads();
     const int t0 = s_t0;
     if (t0 >= nTiles) break;
-    const int t1 = t0 + chunk < nTiles ? t0 + chunk : nTiles;
+    const int t1 = s_t1 < nTiles ? s_t1 : nTiles;
     for (int t = t0; t < t1; t++) {
       const BatchTile tl = tiles[t];
       const int nC = insts[tl.inst].nC;
@@ -167,18 +178,18 @@ __global__ void __launch_bounds__(1024)
         cur = tl.inst;
       }
       const Geom g = insts[tl.inst].g;
-      const int64_t n = tl.end - tl.begin;
+      const int n = (int)(tl.end - tl.begin);
       const uint16_t* lord = nullptr;
+      __syncthreads();  // every wave is done with the previous tile's points
+      if (threadIdx.x == 0) cursor = 0;
       if (sort_off > 0 && n <= kBucketTileMax) {  // (block-uniform)
-        tile_bucket_order<DIM>(pos0, tl.begin, (int)n, g, hist, idx);
+        tile_bucket_order<DIM>(pos0, tl.begin, n, g, hist, idx);
         lord = idx;
+      } else {
+        __syncthreads();
       }
-      const int64_t per = (n + nw - 1) / nw;
-      const int64_t b = tl.begin + (int64_t)w * per;
-      const int64_t e = b + per < tl.end ? b + per : tl.end;
-      if (b < e)
-        integrate_range<DIM, TESS, POW2, 0>(b, e, pos0, out, lds, lds + nC * NE, h, nT, nS, 0, g, nfb_out, 0,
-                                                  lord, tl.begin);
+      integrate_range<DIM, TESS, POW2, 0>(tl.begin, n, &cursor, pos0, out, lds, lds + nC * NE, h, nT, nS, 0, g, nfb_out,
+                                          0, lord);
     }
   }
 }
@@ -206,11 +217,10 @@ __global__ void __launch_bounds__(1024)
                       double h, int nT, int nS, int sort_off) {
   constexpr int NE = DIM * (DIM + 1);
   extern __shared__ double lds[];
-  __shared__ int s_t0;
+  __shared__ int s_t0, cursor;
   // sort_off > 0: each item's points in an order by position (tile_bucket_order)
   unsigned int* hist = reinterpret_cast<unsigned int*>(lds + sort_off);
   uint16_t* idx = reinterpret_cast<uint16_t*>(hist + kBucketMax);
-  const int nw = blockDim.x >> 6, w = threadIdx.x >> 6;
   const double* cur = nullptr;  // Trels in LDS (block-uniform)
   for (;;) {
     __syncthreads();
@@ -234,18 +244,20 @@ __global__ void __launch_bounds__(1024)
         cur = tr;
       }
       const Geom g = it.g;
-      const int64_t n = it.end - it.begin;
-      const uint16_t* lord = nullptr;
-      if (sort_off > 0 && n <= kBucketTileMax) {  // (block-uniform)
-        tile_bucket_order<DIM>(it.pos0, it.begin, (int)n, g, hist, idx);
-        lord = idx;
+      for (int64_t at = it.begin; at < it.end; at += kItemMax) {  // (once, for all but huge items)
+        const int n = it.end - at < kItemMax ? (int)(it.end - at) : kItemMax;
+        const uint16_t* lord = nullptr;
+        __syncthreads();  // every wave is done with the previous points
+        if (threadIdx.x == 0) cursor = 0;
+        if (sort_off > 0 && n <= kBucketTileMax) {  // (block-uniform)
+          tile_bucket_order<DIM>(it.pos0, at, n, g, hist, idx);
+          lord = idx;
+        } else {
+          __syncthreads();
+        }
+        integrate_range<DIM, TESS, POW2, 0>(at, n, &cursor, it.pos0, it.out, lds, lds + nC * NE, h, nT, nS, 0, g,
+                                            nullptr, 0, lord);
       }
-      const int64_t per = (n + nw - 1) / nw;
-      const int64_t b = it.begin + (int64_t)w * per;
-      const int64_t e = b + per < it.end ? b + per : it.end;
-      if (b < e)
-        integrate_range<DIM, TESS, POW2, 0>(b, e, it.pos0, it.out, lds, lds + nC * NE, h, nT, nS, 0, g, nullptr,
-                                                   0, lord, it.begin);
     }
   }
 }
