@@ -1089,16 +1089,19 @@ int items_launch(cpab_ctx* ctx, const WorkItem* items, unsigned int* queue, int 
                  const cpab_batch_sched& q, double h, int nT, int nS) {
   constexpr int NE = DIM * (DIM + 1);
   size_t lds = (size_t)2 * maxNC * NE * sizeof(double);
-  // 1D items of up to kBucketTileMax points are taken in an order by position
+  // 1D runs of up to kBucketTileMax points are taken in an order by position
   // built in LDS after the tables (tile_bucket_order).  Measured on MI355X in
   // the served mix: 1D requests of random points p50 0.49 -> 0.44 ms; the 2D
-  // and 3D requests there are grids whose items are whole rows, already in
-  // an order by position, and the sort's passes made them 1-3 % slower.
-  int sort_off = 0;
-  const size_t lds_sorted = lds + sizeof(unsigned int) * kBucketMax + sizeof(uint16_t) * (size_t)maxLen;
-  if (DIM == 1 && maxLen <= kBucketTileMax && lds_sorted <= (size_t)ctx->max_lds) {
-    sort_off = 2 * maxNC * NE;
-    lds = lds_sorted;
+  // and 3D requests there are grids, whose order tiles or rows give already,
+  // and the sort's passes made them 1-3 % slower.
+  int sort_off = 0, sort_cap = 0;
+  if (DIM == 1 && maxLen <= kBucketTileMax) {
+    sort_cap = maxLen * kGrabMax < kBucketTileMax ? (int)maxLen * kGrabMax : kBucketTileMax;
+    const size_t lds_sorted = lds + sizeof(unsigned int) * kBucketMax + sizeof(uint16_t) * (size_t)sort_cap;
+    if (lds_sorted <= (size_t)ctx->max_lds) {
+      sort_off = 2 * maxNC * NE;
+      lds = lds_sorted;
+    }
   }
   auto k = k_integrate_items<DIM, TESS, POW2>;
   allow_lds(k, lds);
@@ -1110,7 +1113,7 @@ int items_launch(cpab_ctx* ctx, const WorkItem* items, unsigned int* queue, int 
   if (grid > chunks) grid = (int)chunks;
   hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, ctx->stream, queue);
   hipLaunchKernelGGL(k, dim3(grid), dim3(q.block), lds, ctx->stream, items, nItems, q.chunk, queue, h, nT, nS,
-                     sort_off);
+                     sort_off, sort_cap);
   HIP_OK(ctx, hipGetLastError());
   return CPAB_OK;
 }

@@ -617,23 +617,64 @@ __device__ __forceinline__ void advance(double* p, int& c, int& t, int tb, int& 
 // the end of the previous one, of the same p: same value.  Lanes retire and
 // take the next points of the wave's range between calls of `advance`.
 //
-// Processing index i -> point index when the points form a row-major grid
-// of row length w (a multiple of 8): the first nTiled = 8 w floor(nPts / 8 w)
-// indices walk 8 x 8 tiles (64 consecutive indices one tile, the tiles of
-// each band of 8 rows in turn), the rest map to themselves.  A bijection of
-// [0, nPts) whatever w is.
-__device__ __forceinline__ int64_t tile_order(int64_t i, int w, int64_t nTiled) {
-  if (i >= nTiled) return i;
-  const int64_t t = i >> 6;
-  const int u = (int)(i & 63), tpr = w >> 3;
-  const int64_t ty = t / tpr;
-  const int tx = (int)(t - ty * tpr);
-  return (ty * 8 + (u >> 3)) * (int64_t)w + tx * 8 + (u & 7);
+// Processing index i -> point index of n points that form a row-major grid
+// of row length w: bands of r = 1 << lr rows are walked in tiles of r rows and
+// 64 / r columns (64 consecutive indices one tile; w a multiple of 64 / r);
+// what follows the last whole band, from nTiled on, maps to itself.  A
+// bijection of [0, n) whatever w is.
+struct GridOrder {
+  int w = 0, lr = 3;   // w == 0: index order
+  int64_t nTiled = 0;
+  __device__ __forceinline__ int64_t operator()(int64_t i) const {
+    if (i >= nTiled) return i;
+    const int64_t t = i >> 6;
+    const int u = (int)(i & 63), lc = 6 - lr, tpr = w >> lc;
+    const int64_t ty = t / tpr;
+    const int tx = (int)(t - ty * tpr);
+    return ((ty << lr) + (u >> lc)) * (int64_t)w + (tx << lc) + (u & ((1 << lc) - 1));
+  }
+};
+
+// 2D and 3D points that look like a row-major grid (of rows along x) are taken
+// in tiles of x and y: neighbouring points flow alike and cross facets at about the same steps, so a wave's
+// lanes need similar numbers of steps.  The row length is the first index, a
+// multiple of 8 up to 8 x blockDim.x, where y changes from point 0's.  Only
+// the processing order depends on it (every point's result is its own), so a
+// wrong guess costs time only.  In two parts, so that the loads' latency
+// passes while the tables are staged; barriers lie between the parts and
+// after the first store to *w.  On MI355X: 512 x 512 points 80.4 -> 77.1 us in
+// lockstep trips; 3D, 64 x 80 x 96 volume warp 314 -> 292 us (8 x 8 x 1 tiles
+// instead of 64 points of a row).
+template <int DIM>
+struct RowProbe {
+  double y0 = 0.0, yc = 0.0, yp = 0.0;
+  __device__ __forceinline__ void load(const double* __restrict__ pts, int64_t n) {
+    const int64_t i = 8 * ((int64_t)threadIdx.x + 1);
+    if (i < n) {
+      y0 = pts[1];
+      yc = pts[i * DIM + 1];
+      yp = pts[(i - 1) * DIM + 1];
+    }
+  }
+  __device__ __forceinline__ void vote(int64_t n, int* w) const {
+    const int64_t i = 8 * ((int64_t)threadIdx.x + 1);
+    if (i < n && yc != y0 && yp == y0) atomicMin(w, (int)i);
+  }
+};
+
+__device__ __forceinline__ GridOrder grid_order(int w, int64_t n) {
+  GridOrder o;
+  if (w == 0x7fffffff) return o;
+  while (o.lr > 0 && (((int64_t)w << o.lr) > n || (w & ((64 >> o.lr) - 1)) != 0)) o.lr--;
+  if (o.lr == 0) return o;
+  o.w = w;
+  o.nTiled = n / ((int64_t)w << o.lr) * ((int64_t)w << o.lr);
+  return o;
 }
 
 // The block's waves integrate the n points that follow `begin` in the
-// processing order (indices into pos0, out and nfb_out; with gw > 0 through
-// tile_order, with lord through begin + lord[i], a tile's order held in LDS).
+// processing order (indices into pos0, out and nfb_out; with gord.w > 0
+// through it, counted from gbase, with lord through begin + lord[i], a tile's order held in LDS).
 // They draw them from one cursor in LDS (zero at the call, behind a barrier):
 // with a range for each wave the block waited for the one whose points cross
 // the most facets (256 batched instances, 16 waves a block: 11.4 -> 9.6 ms).
@@ -642,14 +683,13 @@ template <int DIM, int TESS, bool POW2, int MODE>
 __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* cursor, const double* __restrict__ pos0,
                                                 double* __restrict__ out, const double* Ttab, const double* Atab,
                                                 double h, int nT, int nS, int64_t nPts, const Geom& g,
-                                                int32_t* __restrict__ nfb_out, int gw = 0,
-                                                const uint16_t* lord = nullptr) {
-  const int64_t nTiled = gw > 0 ? nPts / (8 * (int64_t)gw) * (8 * (int64_t)gw) : 0;
+                                                int32_t* __restrict__ nfb_out, const GridOrder& gord = GridOrder(),
+                                                int64_t gbase = 0, const uint16_t* lord = nullptr) {
   // a grid's tiles are 64 neighbouring points that need similar work, so a
   // wave takes one after another (2048 x 2048 points: 750 -> 610 us); other
   // waves take the next points as soon as kRefill lanes are free (256 batched
   // instances, 8 instead of 16: 14.3 -> 13.9 ms, 32: 16.7; 64: 15.3)
-  const int refill = gw > 0 ? 64 : kRefill;
+  const int refill = gord.w > 0 ? 64 : kRefill;
   double p[DIM];
   int c = 0, t = 0, nfb = 0;
   int64_t my = 0;
@@ -668,7 +708,7 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* curso
       if (!active) {
         const int cand = next + rank_in(idle);
         if (cand < n) {
-          my = gw > 0 ? tile_order(begin + cand, gw, nTiled) : begin + (lord ? (int)lord[cand] : cand);
+          my = gord.w > 0 ? gbase + gord(begin - gbase + cand) : begin + (lord ? (int)lord[cand] : cand);
           active = true;
           load_pt<DIM>(pos0, my, p);
           c = cell_of<DIM, TESS, POW2>(p, g);
@@ -693,26 +733,14 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5)))
                 int32_t* __restrict__ nfb_out, PrepSrc ps) {
   constexpr int NE = DIM * (DIM + 1);
   extern __shared__ double lds[];
-  // calc_T of 2D points: when pos0 looks like a row-major grid, its row
-  // length W (the first index, a multiple of 8 up to 8 x blockDim.x, where y
-  // changes from point 0's), so that waves take 8 x 8 tiles: neighbouring
-  // points flow alike and cross facets at about the same steps, so a wave's
-  // lanes need similar numbers of steps.  Only the processing order depends
-  // on it (every point's result is its own), so a wrong guess costs time
-  // only.  The loads are issued before the tables are staged.
   __shared__ int grid_w, cursor;
-  constexpr bool kDetect = MODE == 0 && DIM == 2;
-  double yc = 0.0, yp = 0.0, y0 = 0.0;
-  const int64_t ic = 8 * ((int64_t)threadIdx.x + 1);
+  constexpr bool kDetect = MODE == 0 && DIM > 1;
+  RowProbe<DIM> probe;
   if (threadIdx.x == 0) {
     grid_w = 0x7fffffff;
     cursor = 0;
   }
-  if (kDetect && ic < nPts) {
-    y0 = pos0[1];
-    yc = pos0[ic * 2 + 1];
-    yp = pos0[(ic - 1) * 2 + 1];
-  }
+  if (kDetect) probe.load(pos0, nPts);
   __syncthreads();
   const double* Ttab = Trels;
   const double* Atab = As;
@@ -722,16 +750,16 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5)))
     Ttab = lds;
     Atab = lds + nC * NE;
   }
-  int gw = 0;
+  GridOrder gord;
   if (kDetect) {
-    if (ic < nPts && yc != y0 && yp == y0) atomicMin(&grid_w, (int)ic);
+    probe.vote(nPts, &grid_w);
     __syncthreads();
-    gw = grid_w != 0x7fffffff && 8 * (int64_t)grid_w <= nPts ? grid_w : 0;
+    gord = grid_order(grid_w, nPts);
   }
   const int per = (int)(blockDim.x >> 6) * ptsPerWave;
   const int64_t begin = (int64_t)blockIdx.x * per;
   const int n = nPts - begin < per ? (int)(nPts - begin) : per;
-  integrate_range<DIM, TESS, POW2, MODE>(begin, n, &cursor, pos0, out, Ttab, Atab, h, nT, nS, nPts, g, nfb_out, gw);
+  integrate_range<DIM, TESS, POW2, MODE>(begin, n, &cursor, pos0, out, Ttab, Atab, h, nT, nS, nPts, g, nfb_out, gord);
 }
 
 // ---------------------------------------------------------- sensitivity
