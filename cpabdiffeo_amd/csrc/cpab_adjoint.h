@@ -25,15 +25,23 @@
 // contribute nothing to the derivative (as in the reference's forward
 // sensitivity solveODE2, calc_2Dto2D.cu:202-319).
 //
-// Schedule, one lane per point: the forward sweep writes the point at the
-// start of every time step to a checkpoint buffer (nT points per point) and,
-// for calc_T, one bit per step recording whether the step was redone; the
-// backward sweep walks the time steps in reverse (each lane its own, for
-// calc_T's map: accepted steps advance together, lanes at a redone step wait
-// for others and run theirs together), recomputes a redone step's nS
-// substep start points from its checkpoint into registers (NSM of them,
-// unrolled so they stay in registers), then runs its substeps' adjoints
-// j = nS-1 .. 0; an accepted step is one Trel adjoint unit.
+// Schedule, one lane per point.  The forward sweep of calc_T's map runs in
+// the two phases of `advance` (steps without a lookup while points stay in
+// their cells, then the redone steps together) and logs events, each a start
+// point, a cell and a count: up to kAdjRun accepted steps in one cell, or one
+// redone step.  The backward sweep takes the events in reverse (each lane its
+// own; lanes at a redone step wait for others and run theirs together),
+// recomputes the points of the steps or substeps from the event's start point
+// into registers and runs their adjoints back over them; the last lane with
+// events left spreads them over its wave.  calc_T_simple's map logs the start
+// point of every time step, and every step is a redone one.
+//
+// What bounds it: FP64 instructions (each wave's redone steps cost ~1 900 a
+// pass, its accepted ones ~50 a step), and below ~20 pairs of 128 x 128
+// pixels the corner's pixel alone, one chain of nT nS substeps.  64 pairs of
+// 128 x 128, 100 steps, 10 substeps: 1.72 ms with a checkpoint, a lookup and
+// a dependent load for every step, 1.03 with events, 0.69 with the last lane's
+// events spread (4 pairs: 0.97, 0.97 and 0.46).
 //
 // Accumulation, bit-reproducible: each lane keeps two register
 // accumulators, dJ/dA of its current RK2 cell and dJ/dTrel of its current
@@ -70,9 +78,8 @@ struct AdjDesc {
   const float* src;      // MODE 1: (nInst, H, W)
   const float* dst;      // MODE 1: (nInst, H, W)
   uint32_t* sig;         // optional (nInst, nPts): hash of every cell the forward sweep looked up
-  double* ckpt;          // (nInst, nT, nPts, 2) workspace
-  uint64_t* redo_bits;   // calc_T map: (nInst, ceil(nT / 64), nPts) workspace, bit k % 64 of word k / 64:
-                         // step k was redone by RK2
+  double* ckpt;          // (nInst, nT, nPts, 2) workspace: start points of the steps (calc_T map: of the events)
+  uint16_t* event;       // calc_T map: (nInst, nT, nPts) workspace, the events (adj_event)
   double* partial;       // (nInst, blocks per instance, NG*nC*6 + 2): tables, loss, redone steps
   double h;
   int nT, nS;
@@ -103,6 +110,18 @@ __device__ __forceinline__ double sample2_grad(const float* __restrict__ img, in
   *gy_out = b - a;
   return gy * a + fy * b;
 }
+
+// An event of the forward sweep of calc_T's map: its cell and its count of
+// accepted steps, 0 for one redone step.  16 bits: the tables' place in LDS
+// keeps nC below 854.
+__device__ __forceinline__ uint16_t adj_event(int cell, int n) { return (uint16_t)(cell | (n << 10)); }
+__device__ __forceinline__ int adj_cell(int ev) { return ev & 1023; }
+__device__ __forceinline__ int adj_steps(int ev) { return ev >> 10; }
+// Accepted steps an event holds at most (64 pairs of 128 x 128: 6 steps 753 us,
+// 8 718, 10 709; more do not fit the registers), and runs between two redo
+// phases of the forward sweep (5 the same, 10: 755).
+constexpr int kAdjRun = 10;
+constexpr int kAdjSegs = 3;
 
 __device__ __forceinline__ uint32_t sig_mix(uint32_t s, int c) { return s * 0x9E3779B1u + (uint32_t)(c + 1); }
 
@@ -137,6 +156,18 @@ __device__ __forceinline__ int rk2_substep_in(double* p, int c, const double* At
   return cell2<TESS, POW2>(p, g);
 }
 
+// The value of `v` on lane i (wave-uniform).
+__device__ __forceinline__ double lane_value(double v, int i) {
+  union {
+    double d;
+    int w[2];
+  } u;
+  u.d = v;
+  u.w[0] = __builtin_amdgcn_readlane(u.w[0], i);
+  u.w[1] = __builtin_amdgcn_readlane(u.w[1], i);
+  return u.d;
+}
+
 // Active lanes with `need` add their accumulator G into row `cell` of the
 // wave's table `tab`, one lane at a time in lane order.  Which lanes are
 // active where the call sits is fixed by the data and the code, so the order
@@ -149,7 +180,8 @@ __device__ __forceinline__ void adj_flush(bool need, int cell, const double* G, 
     if (lane == l) {
       double* t = tab + cell * 6;
 #pragma unroll
-      for (int e = 0; e < 6; e++) t[e] = t[e] + G[e];
+      for (int e = 0; e < 6; e++)
+        __hip_atomic_fetch_add(t + e, G[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     __builtin_amdgcn_wave_barrier();
     m &= m - 1;
@@ -216,37 +248,81 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
       p[0] = (double)(pix % D.W);
       p[1] = (double)(pix / D.W);
     }
-    // forward sweep, one checkpoint per time step (and, for calc_T, the
-    // step's decision, 64 steps to a word)
     double* ck = D.ckpt + (int64_t)inst * nT * nPts * 2;
-    const int nWords = (nT + 63) >> 6;
-    uint64_t* rb = FWD ? D.redo_bits + (int64_t)inst * nWords * nPts : nullptr;
+    uint16_t* evs = FWD ? D.event + (int64_t)inst * nT * nPts : nullptr;
     uint32_t sg = 0;
-    uint64_t bits = 0;
     // the cell of p, carried: an accepted step ends in the cell it started
     // in, and each substep looks up the cell of its end point
     int c = cell2<TESS, POW2>(p, g);
-    for (int k = 0; k < nT; k++) {
-      ck[((int64_t)k * nPts + idx) * 2] = p[0];
-      ck[((int64_t)k * nPts + idx) * 2 + 1] = p[1];
-      bool redo = true;
-      if (FWD) {
-        double pn[2];
-        affine<2>(pn, Tr + c * 6, p);
-        const int cn = cell2<TESS, POW2>(pn, g);
-        sg = sig_mix(sig_mix(sg, c), cn);
-        redo = cn != c;
-        if (!redo) {
-          p[0] = pn[0];
-          p[1] = pn[1];
+    int nev = 0;  // events logged
+    if (FWD) {
+      // Forward sweep of calc_T's map in the two phases of `advance`; logged
+      // are events, each with its start point: up to NSM accepted steps, or
+      // one redone step.
+      const bool has_sig = D.sig != nullptr;
+      auto log_start = [&](const double* q) {
+        *reinterpret_cast<double2*>(ck + ((int64_t)nev * nPts + idx) * 2) = make_double2(q[0], q[1]);
+      };
+      auto log_event = [&](int cell, int n) { evs[(int64_t)nev++ * nPts + idx] = adj_event(cell, n); };
+      int t = 0, cool = 0;
+      for (;;) {
+        const uint64_t todo = ballot(t < nT);
+        if (todo == 0) break;
+        bool waits = t < nT;
+        if (cool > 0) {
+          cool--;
+        } else {
+          CellBounds<2, TESS> B;
+          double R[6];
+#pragma unroll
+          for (int e = 0; e < 6; e++) R[e] = Tr[c * 6 + e];
+          B.enter(p, c, g);
+          uint64_t go = B.inside(p, g) & todo;
+          if (go == 0) cool = 8;
+          for (int s = 0; s < kAdjSegs && go != 0; s++) {
+            const bool runs = lane_in(go);
+            const int t0 = t, lim = nT - t < kAdjRun ? nT : t + kAdjRun;
+            if (runs) log_start(p);
+            while (go != 0) {
+              double y[2];
+              affine<2>(y, R, p);
+              go &= B.inside(y, g) & lanes_lt(t, lim);
+              const bool in = lane_in(go);
+              p[0] = in ? y[0] : p[0];
+              p[1] = in ? y[1] : p[1];
+              if (has_sig) sg = in ? sig_mix(sig_mix(sg, c), c) : sg;
+              t += in ? 1 : 0;
+            }
+            if (t > t0) log_event(c, t - t0);
+            if (runs) waits = t < lim;
+            go = ballot(runs && t == lim && t < nT);
+          }
         }
-        bits |= (uint64_t)redo << (k & 63);
-        if ((k & 63) == 63 || k == nT - 1) {
-          rb[(int64_t)(k >> 6) * nPts + idx] = bits;
-          bits = 0;
+        if (waits) {
+          double pn[2];
+          affine<2>(pn, Tr + c * 6, p);
+          const int cn = cell2<TESS, POW2, true>(pn, g);
+          sg = sig_mix(sig_mix(sg, c), cn);
+          log_start(p);
+          if (cn == c) {
+            log_event(c, 1);
+            p[0] = pn[0];
+            p[1] = pn[1];
+          } else {
+            log_event(c, 0);
+            nredo++;
+            for (int j = 0; j < nS; j++) {
+              sg = sig_mix(sg, c);
+              c = rk2_substep_in<TESS, POW2>(p, c, At, h, g);
+            }
+          }
+          t++;
         }
       }
-      if (redo) {
+    } else {  // calc_T_simple's map: a checkpoint a time step, every step nS substeps
+      for (int k = 0; k < nT; k++) {
+        ck[((int64_t)k * nPts + idx) * 2] = p[0];
+        ck[((int64_t)k * nPts + idx) * 2 + 1] = p[1];
         nredo++;
         for (int j = 0; j < nS; j++) {
           sg = sig_mix(sg, c);
@@ -274,10 +350,6 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
     }
     // backward sweep
     int ca = -1, ct = -1;  // cells of the RK2 and Trel accumulators (-1: empty)
-    // the cell of the end point of the step being processed, carried back:
-    // an accepted step starts in the cell it ends in, and a redone step's
-    // start cell is the one its first substep looks up
-    int cq = c;
     double Ga[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     double Gt[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     // the substeps' start cells as the recompute looks them up, two 16-bit
@@ -287,7 +359,7 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
     constexpr bool kKeepCells = NSM <= 10;
     // One redone step from its start point q, in reverse: the recompute of
     // its substep start points (and cells), then the adjoint of each
-    // substep.  Sets cq to the cell of q.
+    // substep.
     auto redone_step = [&](const double* q) {
       double ps[NSM][2];
       uint32_t cs[(NSM + 1) / 2];
@@ -308,7 +380,6 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
         if (j < nS) {
           const double* pj = ps[j];
           const int c = kKeepCells ? (int)((cs[j >> 1] >> ((j & 1) * 16)) & 0xffffu) : cell2<TESS, POW2>(pj, g);
-          if (j == 0) cq = c;
           adj_flush(ca >= 0 && c != ca, ca, Ga, GA);
           if (c != ca) {
 #pragma unroll
@@ -335,56 +406,139 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
       }
     };
     if (FWD) {
-      // Each lane walks its own steps back.  A trip either takes one
-      // accepted step on every lane whose current step is accepted, or
-      // (a redo trip) runs the redone step of every lane parked at one;
-      // redo trips run once kRedoBatch lanes are parked or nothing else can
-      // move, so a redone step costs its wave one pass of its nS substeps
-      // shared by several lanes rather than one pass per lane and step.
-      // Every choice is a ballot of the data: the sums keep a fixed order.
-      // (12 lanes measured best on MI355X: 6, 8 and 16 within 4 %.)
-      constexpr int kRedoBatch = 12;
-      int k = nT - 1;  // this lane's step (-1: done)
-      double q[2] = {ck[((int64_t)k * nPts + idx) * 2], ck[((int64_t)k * nPts + idx) * 2 + 1]};
-      bits = rb[(int64_t)(k >> 6) * nPts + idx];
-      bool redo = (bits >> (k & 63)) & 1;
-      auto next_step = [&]() {  // the step before: its start point (checkpoint) and decision bit
-        if (--k >= 0) {
-          q[0] = ck[((int64_t)k * nPts + idx) * 2];
-          q[1] = ck[((int64_t)k * nPts + idx) * 2 + 1];
-          if ((k & 63) == 63) bits = rb[(int64_t)(k >> 6) * nPts + idx];
-          redo = (bits >> (k & 63)) & 1;
+      // Each lane walks its own events back.  A trip either takes one event
+      // of accepted steps on every lane whose current event is one, or (a
+      // redo trip) the redone step of every lane parked at one; redo trips
+      // run once kRedoBatch lanes are parked or nothing else can move, so a
+      // redone step costs its wave one pass of its nS substeps shared by
+      // several lanes rather than one pass per lane and step.  Every choice
+      // is a ballot of the data: the sums keep a fixed order.
+      //
+      // The last lane with events left (beside a corner of the domain a point
+      // can redo all its steps while its neighbours are long done) spreads
+      // them over the wave: each lane takes one, finds the matrix that
+      // carries lambda over it, and with lambda carried to every event the
+      // events are taken like any others, all at once.
+      constexpr int kRedoBatch = 24;  // 64 pairs of 128 x 128: 8 lanes 730 us, 12 709, 20 678, 32 678, 64 687
+      constexpr int kTailMin = 3;     // events that are worth a tail (12: the same)
+      const int lane = threadIdx.x & 63, nAct = __popcll(__builtin_amdgcn_read_exec());
+      bool tail = false;   // (wave-uniform)
+      int eT = -1;         // the tail's events left
+      int L = 0;           // the lane whose events the tail takes
+      double lx = 0.0, ly = 0.0;  // the tail's lambda behind event eT
+      int e = nev - 1;     // this lane's event (-1: done)
+      double2 q2 = make_double2(0.0, 0.0);
+      int ev = 0;
+      auto load_event = [&]() {
+        if (e >= 0) {
+          const int64_t pt = tail ? idx - lane + L : idx;
+          q2 = *reinterpret_cast<const double2*>(ck + ((int64_t)e * nPts + pt) * 2);
+          ev = evs[(int64_t)e * nPts + pt];
         }
       };
+      load_event();
       for (;;) {
-        const uint64_t parked = __ballot(k >= 0 && redo);
-        const uint64_t ready = __ballot(k >= 0 && !redo);
-        if ((parked | ready) == 0) break;
-        if (ready == 0 || __popcll(parked) >= kRedoBatch) {
-          if (k >= 0 && redo) {
-            redone_step(q);
-            next_step();
+        const bool redo = adj_steps(ev) == 0;
+        const uint64_t parked = ballot(e >= 0 && redo);
+        const uint64_t ready = ballot(e >= 0 && !redo);
+        const uint64_t left = parked | ready;
+        if (left == 0 && eT < 0) break;
+        bool fill = left == 0;  // the tail's next events
+        if (!tail && __popcll(left) == 1) {
+          L = __builtin_ctzll(left);
+          const int eL = __builtin_amdgcn_readlane(e, L);
+          if (eL + 1 >= kTailMin) {
+            fill = tail = true;
+            eT = eL;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // (lane L's log, read by the others)
+            lx = lane_value(lam[0], L);
+            ly = lane_value(lam[1], L);
           }
-        } else if (k >= 0 && !redo) {  // the accepted Trel step: it starts in the cell it ends in
-          const int c0 = cq;
+        }
+        if (fill) {
+          e = eT - lane;
+          load_event();
+          double P[4] = {1.0, 0.0, 0.0, 1.0};  // lambda before the event = P lambda behind it
+          if (e >= 0) {
+            const int c0 = adj_cell(ev), n = adj_steps(ev);
+            double r[2] = {q2.x, q2.y};
+            const int steps = n == 0 ? nS : n;
+            for (int j = 0; j < steps; j++) {
+              double M[4];
+              if (n == 0) {
+                const double* A = At + rk2_substep<TESS, POW2>(r, At, h, g) * 6;
+                const double a = h * A[0], b = h * A[3], d = h * A[1], f = h * A[4];
+                M[0] = 1.0 + (a + 0.5 * __builtin_fma(a, a, b * d));
+                M[1] = b + 0.5 * __builtin_fma(a, b, b * f);
+                M[2] = d + 0.5 * __builtin_fma(d, a, f * d);
+                M[3] = 1.0 + (f + 0.5 * __builtin_fma(d, b, f * f));
+              } else {
+                const double* T = Tr + c0 * 6;
+                M[0] = T[0];
+                M[1] = T[3];
+                M[2] = T[1];
+                M[3] = T[4];
+              }
+              const double p0 = __builtin_fma(P[0], M[0], P[1] * M[2]);
+              const double p2 = __builtin_fma(P[2], M[0], P[3] * M[2]);
+              P[1] = __builtin_fma(P[0], M[1], P[1] * M[3]);
+              P[3] = __builtin_fma(P[2], M[1], P[3] * M[3]);
+              P[0] = p0;
+              P[2] = p2;
+            }
+          }
+          const int nB = eT + 1 < nAct ? eT + 1 : nAct;
+          for (int i = 0; i < nB; i++) {
+            if (lane == i) {
+              lam[0] = lx;
+              lam[1] = ly;
+            }
+            const double x = __builtin_fma(lane_value(P[0], i), lx, lane_value(P[1], i) * ly);
+            ly = __builtin_fma(lane_value(P[2], i), lx, lane_value(P[3], i) * ly);
+            lx = x;
+          }
+          eT -= nB;
+          continue;
+        }
+        if (ready == 0 || __popcll(parked) >= kRedoBatch) {
+          if (e >= 0 && redo) {
+            const double q[2] = {q2.x, q2.y};
+            e = tail ? -1 : e - 1;
+            load_event();  // (in flight while the step is processed)
+            redone_step(q);
+          }
+        } else if (e >= 0 && !redo) {  // accepted steps, all in one cell
+          const int c0 = adj_cell(ev), n = adj_steps(ev);
+          double qs[kAdjRun][2];
+          qs[0][0] = q2.x;
+          qs[0][1] = q2.y;
+          e = tail ? -1 : e - 1;
+          load_event();
           adj_flush(ct >= 0 && c0 != ct, ct, Gt, GT);
           if (c0 != ct) {
 #pragma unroll
-            for (int e = 0; e < 6; e++) Gt[e] = 0.0;
+            for (int i = 0; i < 6; i++) Gt[i] = 0.0;
             ct = c0;
           }
-          const double* T = Tr + c0 * 6;
-          Gt[0] += lam[0] * q[0];
-          Gt[1] += lam[0] * q[1];
-          Gt[2] += lam[0];
-          Gt[3] += lam[1] * q[0];
-          Gt[4] += lam[1] * q[1];
-          Gt[5] += lam[1];
-          const double l0 = T[0] * lam[0] + T[3] * lam[1];
-          const double l1 = T[1] * lam[0] + T[4] * lam[1];
-          lam[0] = l0;
-          lam[1] = l1;
-          next_step();
+          double T[6];
+#pragma unroll
+          for (int i = 0; i < 6; i++) T[i] = Tr[c0 * 6 + i];
+#pragma unroll
+          for (int j = 1; j < kAdjRun; j++) affine<2>(qs[j], T, qs[j - 1]);  // (past n: not used)
+#pragma unroll
+          for (int j = kAdjRun - 1; j >= 0; j--) {
+            if (j < n) {
+              Gt[0] = __builtin_fma(lam[0], qs[j][0], Gt[0]);
+              Gt[1] = __builtin_fma(lam[0], qs[j][1], Gt[1]);
+              Gt[2] += lam[0];
+              Gt[3] = __builtin_fma(lam[1], qs[j][0], Gt[3]);
+              Gt[4] = __builtin_fma(lam[1], qs[j][1], Gt[4]);
+              Gt[5] += lam[1];
+              const double l0 = __builtin_fma(T[0], lam[0], T[3] * lam[1]);
+              lam[1] = __builtin_fma(T[1], lam[0], T[4] * lam[1]);
+              lam[0] = l0;
+            }
+          }
         }
       }
     } else {  // calc_T_simple's map: every step is nS substeps, the same on every lane

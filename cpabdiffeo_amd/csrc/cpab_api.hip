@@ -665,7 +665,7 @@ int adjoint2d(cpab_ctx* ctx, int mode, int tess, int nC, int nInst, int64_t nPts
   int r = make_geom(ctx, 2, tess, nC0, nC1, 0, ix, iy, 1.0, &g, &pow2);
   if (r) return r;
   if ((r = check_nC(ctx, 2, tess, nC, nC0, nC1, 0))) return r;
-  // (the tables' LDS bound below keeps nC far lower; the kernel packs cells in 16 bits)
+  // (the tables' LDS bound below keeps nC lower; the kernel packs cells in 16 bits, for the calc_T map in 10)
   if (nC > 65535) return fail(ctx, CPAB_ERR_UNSUPPORTED, "the adjoint takes at most 65535 cells");
   if (nInst < 1 || nInst > 65535) return fail(ctx, CPAB_ERR_ARG, "nInst must be in [1, 65535]");
   if (nPts < 0 || nT < 0 || nS < 0) return fail(ctx, CPAB_ERR_ARG, "bad sizes");
@@ -677,7 +677,7 @@ int adjoint2d(cpab_ctx* ctx, int mode, int tess, int nC, int nInst, int64_t nPts
   int waves = 4;
   while (waves > 1 && adj_lds_doubles(nC, fwd, waves) * sizeof(double) > (size_t)ctx->max_lds) waves >>= 1;
   const size_t lds = adj_lds_doubles(nC, fwd, waves) * sizeof(double);
-  if (lds > (size_t)ctx->max_lds) return fail(ctx, CPAB_ERR_UNSUPPORTED, "tables exceed LDS");
+  if (lds > (size_t)ctx->max_lds || (fwd && nC > 1023)) return fail(ctx, CPAB_ERR_UNSUPPORTED, "tables exceed LDS");
   if (nPts == 0 || nT == 0) {  // the identity map: zero gradient (and loss of the unwarped images in MODE 1)
     if (mode == 1) return fail(ctx, CPAB_ERR_UNSUPPORTED, "empty integration in the SSD adjoint");
     HIP_OK(ctx, hipMemsetAsync(gradA, 0, sizeof(double) * NT * nInst, ctx->stream));
@@ -691,7 +691,7 @@ int adjoint2d(cpab_ctx* ctx, int mode, int tess, int nC, int nInst, int64_t nPts
   if (nbx > 0x7fffffffLL) return fail(ctx, CPAB_ERR_ARG, "too many points");
   const size_t ck = (size_t)nInst * nT * nPts * 2, pa = (size_t)nInst * nbx * (NG * NT + 2);
   const size_t gt = fwd ? (size_t)nInst * NT : 0;
-  const size_t rb = fwd ? (size_t)nInst * ((nT + 63) / 64) * nPts : 0;  // 64-bit words
+  const size_t rb = fwd ? ((size_t)nInst * nT * nPts + 3) / 4 : 0;  // the events, 16 bits each
   if ((r = ensure_ws(ctx, (ck + pa + gt + rb) * sizeof(double)))) return r;
   AdjDesc D{};
   D.nInst = nInst;
@@ -709,7 +709,7 @@ int adjoint2d(cpab_ctx* ctx, int mode, int tess, int nC, int nInst, int64_t nPts
   D.sig = sig;
   D.ckpt = ctx->ws;
   D.partial = ctx->ws + ck;
-  D.redo_bits = fwd ? reinterpret_cast<uint64_t*>(ctx->ws + ck + pa + gt) : nullptr;
+  D.event = fwd ? reinterpret_cast<uint16_t*>(ctx->ws + ck + pa + gt) : nullptr;
   const bool ns10 = nS <= 10;  // the substep starts of a redone step in 10 registers pairs, else 16
   D.h = dt / (double)nS;
   D.nT = nT;
