@@ -133,6 +133,8 @@ int make_geom(cpab_ctx* ctx, int dim, int tess, int nC0, int nC1, int nC2, doubl
     rmax = 1.0 / inc[d] > rmax ? 1.0 / inc[d] : rmax;
   }
   g->eps = (nmax + 16.0) * 0x1p-46 + 2e-10 * rmax;
+  g->sc1 = 1.0 / (1.0 - 2.0 * g->eps);
+  g->sc17 = 1.0 / (17.0 - g->eps);
   // The type I clamps must leave a non-empty range, or the box index of a
   // clamped point would be negative.
   if (tess == TESS_I && !(g->top_x > 0.0 && g->top_y > 0.0 && (dim < 3 || g->top_z > 0.0)))
@@ -510,31 +512,26 @@ int cpab_calc_grad_theta(cpab_ctx* ctx, int dim, int tess, int nC, const double*
   if (overlap(pos0, pb, pos, pb)) return fail(ctx, CPAB_ERR_ALIAS, "pts and out cannot point to the same memory");
   const int64_t steps64 = (int64_t)nS * nT;
   if (steps64 > 0x7fffffffLL) return fail(ctx, CPAB_ERR_ARG, "nStepsODE*nTimeSteps overflows int");
-  const int ne = dim * (dim + 1);
   const double h = dt / (double)nS;
-  // columns per thread: 8 when As + 8 basis tables fit in LDS, else 2, else
-  // 2 with the tables read from global memory
-  const size_t lds8 = (size_t)9 * nC * ne * sizeof(double), lds2 = (size_t)3 * nC * ne * sizeof(double);
-  const int jc = lds8 <= (size_t)ctx->max_lds ? 8 : 2;
-  const bool in_lds = jc == 8 || lds2 <= (size_t)ctx->max_lds;
-  const size_t lds = !in_lds ? 0 : (jc == 8 ? lds8 : lds2);
+  // Columns a thread: as many as its registers hold with their rows (8, in 3D
+  // 4), fewer when that leaves most of the chip's SIMDs without a wave, which
+  // the chain of substeps then costs more than the point's own share of it
+  // (62 columns: 2 000 points, 8 a thread 667 us, 4 400, 2 278; 500 points
+  // 669, 398, 264, 1: 197; 8 000 points, 1 000 waves of 8: 744, 4: 813).
+  const int64_t waves = (nPts + 63) / 64;
+  int jc = dim == 3 ? 4 : 8;
+  while (jc > 1 && waves * ((d + jc - 1) / jc) < 3 * (int64_t)ctx->n_cu) jc >>= 1;
   const dim3 grid((unsigned)((nPts + 255) / 256), (unsigned)((d + jc - 1) / jc));
+#define GRAD_RUN(J_)                                                                                         \
+  hipLaunchKernelGGL((k_grad_theta<D_, T_, P_, J_>), grid, dim3(256), 0, ctx->stream, pos0, pos, As, Bs, grad, \
+                     d, h, (int)steps64, nPts, g, nC)
   DISPATCH_GEOM(dim, tess, pow2, {
-    if (jc == 8) {
-      auto k = k_grad_theta<D_, T_, P_, 8, true>;
-      allow_lds(k, lds);
-      hipLaunchKernelGGL(k, grid, dim3(256), lds, ctx->stream, pos0, pos, As, Bs, grad, d, h, (int)steps64, nPts,
-                         g, nC);
-    } else if (in_lds) {
-      auto k = k_grad_theta<D_, T_, P_, 2, true>;
-      allow_lds(k, lds);
-      hipLaunchKernelGGL(k, grid, dim3(256), lds, ctx->stream, pos0, pos, As, Bs, grad, d, h, (int)steps64, nPts,
-                         g, nC);
-    } else {
-      hipLaunchKernelGGL((k_grad_theta<D_, T_, P_, 2, false>), grid, dim3(256), 0, ctx->stream, pos0, pos, As, Bs,
-                         grad, d, h, (int)steps64, nPts, g, nC);
-    }
+    if (jc == 8) GRAD_RUN((D_ == 3 ? 4 : 8));
+    else if (jc == 4) GRAD_RUN(4);
+    else if (jc == 2) GRAD_RUN(2);
+    else GRAD_RUN(1);
   });
+#undef GRAD_RUN
   HIP_OK(ctx, hipGetLastError());
   return CPAB_OK;
 }

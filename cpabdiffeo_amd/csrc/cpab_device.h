@@ -38,6 +38,7 @@ struct Geom {
   double top_x, top_y, top_z;     // clamps nC0*inc_x-1e-10, nC1*inc_y-1e-10, nC2*inc_x-1e-10
   double wall_x, wall_y;          // nC0*inc_x, nC1*inc_y (2D type I out-of-domain tests)
   double eps;                     // margin of CellBounds, in increments
+  double sc1, sc17;               // 1 / (1 - 2 eps), 1 / (17 - eps): its scales (2D type I)
 };
 
 __device__ __forceinline__ double dmin(double a, double b) { return __builtin_fmin(a, b); }

@@ -345,10 +345,11 @@ struct CellBounds<2, TESS_I> {
     const bool onwall = at == (b2 ? last : 0.0);  // (right and bottom look at the far wall)
     const bool usex = side != onwall;
     const double o = usex ? i : j, olast = usex ? ni : nj;
-    const double lo = onwall & (o == 0.0) ? -16.0 : o + g.eps;
-    const double hi = onwall & (o == olast) ? olast + 17.0 : o + 1.0 - g.eps;
-    // |w| < 1/2 for lo < s < hi
-    const double sc = 1.0 / (hi - lo);
+    const bool first = onwall & (o == 0.0), end = onwall & (o == olast);
+    const double lo = first ? -16.0 : o + g.eps;
+    const double hi = end ? olast + 17.0 : o + 1.0 - g.eps;
+    // |w| < 1/2 for lo < s < hi; sc = 1 / (hi - lo)
+    const double sc = first & end ? 1.0 / 33.0 : first | end ? g.sc17 : g.sc1;
     ax = usex ? g.rinc_x * sc : 0.0;
     by = usex ? 0.0 : g.rinc_y * sc;
     mid = -0.5 * (lo + hi) * sc;
@@ -766,69 +767,80 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5)))
 // calc_grad_theta (cpab/gpu/calc_2Dto2D.cu:202-319, 448-491): calc_T_simple
 // together with the forward sensitivity q_j = dp/dtheta_j of every basis
 // column j, integrated by the same RK2 (q' = B_j [p;1] + A_lin q).  Grid
-// (point blocks, column chunks): a thread owns one point and JC columns,
-// whose basis tables (layout (d, nC, DIM, DIM+1)) sit in LDS with As; the
+// (point blocks, column chunks): a thread owns one point and JC columns; the
 // reference keeps q in global memory and re-reads it every substep, here it
-// stays in registers (same values).  Output grad (nPts, DIM, d) and, from
-// the first chunk, the end points.  JC = columns per thread (the widest
-// whose tables fit in LDS); LDS = false reads the tables from global memory.
-template <int DIM, int TESS, bool POW2, int JC, bool LDS>
-__global__ void __launch_bounds__(256)
+// stays in registers (same values), and so do the cell's row and the columns'
+// basis rows (layout (d, nC, DIM, DIM+1)), read again when the point has left
+// the cell.  Output grad (nPts, DIM, d) and, from the first chunk, the end
+// points.  The last chunk ends at column d: it repeats columns of the one
+// before where JC does not divide d (the same values).
+//
+// Bound by FP64 instructions without FMA, 38 a substep and column and 48 a
+// substep; no branch between the columns, whose LDS reads each stalled the
+// wave when the rows were read every substep (and staged: now a wave reads
+// rows on the ~1/4 of its substeps in which some point changes cell, and from
+// LDS that measured the same).  128 x 128 grid, 62 columns: 1.86 -> 1.63 ms
+// (0.25 of it the corner's pixel, which changes cell every substep); 16 384
+// random points 2.79 -> 1.35 ms (28 T instructions/s of the 39 that two waves
+// a SIMD can issue), 2 000: 1.55 -> 0.31, 500: 1.55 -> 0.20.
+template <int DIM, int TESS, bool POW2, int JC>
+__global__ void __launch_bounds__(256, 2)
     k_grad_theta(const double* __restrict__ pos0, double* __restrict__ pos, const double* __restrict__ As,
                  const double* __restrict__ Bs, double* __restrict__ grad, int d, double h, int nSteps,
                  int64_t nPts, Geom g, int nC) {
   constexpr int NE = DIM * (DIM + 1);
-  extern __shared__ double lds[];
-  const int j0 = blockIdx.y * JC;
-  const int nj = d - j0 < JC ? d - j0 : JC;
-  const double* Al = As;
+  const int jc = (int)blockIdx.y * JC, j0 = jc + JC <= d ? jc : (d > JC ? d - JC : 0);
+  const int nj = d < JC ? d : JC;
   const double* Bl = Bs + (int64_t)j0 * nC * NE;
-  if (LDS) {
-    double* a = lds;
-    double* b = lds + nC * NE;
-    for (int i = threadIdx.x; i < nC * NE; i += blockDim.x) a[i] = As[i];
-    for (int i = threadIdx.x; i < nj * nC * NE; i += blockDim.x) b[i] = Bs[(int64_t)j0 * nC * NE + i];
-    __syncthreads();
-    Al = a;
-    Bl = b;
-  }
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= nPts) return;
-  double p[DIM], v[DIM], pMid[DIM], vMid[DIM];
-  double q[JC][DIM];
+  const double hh = h * 0.5;  // (as in `advance`)
+  double p[DIM], q[JC][DIM], A[NE], B[JC][NE];
 #pragma unroll
   for (int jj = 0; jj < JC; jj++)
 #pragma unroll
     for (int i = 0; i < DIM; i++) q[jj][i] = 0.0;
   load_pt<DIM>(pos0, idx, p);
+  CellBounds<DIM, TESS> bounds;
+  const uint64_t all = __builtin_amdgcn_read_exec();
+  uint64_t in = 0;  // lanes whose point is in the cell of their rows
+  int c = -1;
   for (int s = 0; s < nSteps; s++) {
-    const int c = cell_of<DIM, TESS, POW2>(p, g);
-    const double* A = Al + c * NE;
+    if (in != all) {
+      if (!lane_in(in)) {
+        const int cn = cell_of<DIM, TESS, POW2>(p, g);
+        if (cn != c) {
+          c = cn;
+#pragma unroll
+          for (int e = 0; e < NE; e++) A[e] = As[c * NE + e];
+#pragma unroll
+          for (int jj = 0; jj < JC; jj++)
+#pragma unroll
+            for (int e = 0; e < NE; e++) B[jj][e] = Bl[((jj < nj ? jj : 0) * nC + c) * NE + e];
+        }
+      }
+      bounds.enter(p, c, g);
+    }
+    double v[DIM], pMid[DIM];
     affine<DIM>(v, A, p);
 #pragma unroll
-    for (int i = 0; i < DIM; i++) pMid[i] = p[i] + h * v[i] / 2.;
-    affine<DIM>(vMid, A, pMid);
+    for (int i = 0; i < DIM; i++) pMid[i] = p[i] + hh * v[i];
+    affine<DIM>(v, A, pMid);
 #pragma unroll
     for (int jj = 0; jj < JC; jj++) {
-      if (jj < nj) {
-        const double* Bj = Bl + (jj * nC + c) * NE;
-        double BtT[DIM], AdT[DIM], u[DIM], qMid[DIM];
-        affine<DIM>(BtT, Bj, p);
-        linear<DIM>(AdT, A, q[jj]);
+      double BtT[DIM], AdT[DIM], qMid[DIM];
+      affine<DIM>(BtT, B[jj], p);
+      linear<DIM>(AdT, A, q[jj]);
 #pragma unroll
-        for (int i = 0; i < DIM; i++) u[i] = BtT[i] + AdT[i];
+      for (int i = 0; i < DIM; i++) qMid[i] = q[jj][i] + hh * (BtT[i] + AdT[i]);
+      affine<DIM>(BtT, B[jj], pMid);
+      linear<DIM>(AdT, A, qMid);
 #pragma unroll
-        for (int i = 0; i < DIM; i++) qMid[i] = q[jj][i] + h * u[i] / 2.;
-        affine<DIM>(BtT, Bj, pMid);
-        linear<DIM>(AdT, A, qMid);
-#pragma unroll
-        for (int i = 0; i < DIM; i++) u[i] = BtT[i] + AdT[i];
-#pragma unroll
-        for (int i = 0; i < DIM; i++) q[jj][i] += u[i] * h;
-      }
+      for (int i = 0; i < DIM; i++) q[jj][i] += (BtT[i] + AdT[i]) * h;
     }
 #pragma unroll
-    for (int i = 0; i < DIM; i++) p[i] += vMid[i] * h;
+    for (int i = 0; i < DIM; i++) p[i] += v[i] * h;
+    in = bounds.inside(p, g);
   }
   if (blockIdx.y == 0) store_pt<DIM>(pos, idx, p);
 #pragma unroll
@@ -838,7 +850,12 @@ __global__ void __launch_bounds__(256)
       for (int i = 0; i < DIM; i++) grad[(idx * DIM + i) * d + j0 + jj] = q[jj][i];
 }
 
-// calc_T_simple: nStepsODE * nTimeSteps RK2 substeps (calc_2Dto2D.cu:412-445).
+// calc_T_simple: nStepsODE * nTimeSteps RK2 substeps (calc_2Dto2D.cu:412-445),
+// with a lookup only where some point of the wave has left the bounds of its
+// cell.  Bound by FP64 instructions: 35 a substep and point where a lookup in
+// each took 75 and a table read.  1 000 points 232 -> 150 us; 250 000: 2D type
+// I 640 -> 335, type II 470 -> 263, 3 x 5 cells 1 283 -> 395, 3D (100 000)
+// 850 -> 375; 512 x 512 grid 535 -> 480, all of it the corner's wave.
 template <int DIM, int TESS, bool POW2, bool LDS>
 __global__ void __launch_bounds__(1024)
     k_simple(const double* __restrict__ pos0, double* __restrict__ out, const double* __restrict__ As,
@@ -853,16 +870,26 @@ __global__ void __launch_bounds__(1024)
   }
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nPts) return;
-  double p[DIM], y[DIM], m[DIM];
+  const double hh = h * 0.5;  // (as in `advance`)
+  double p[DIM], y[DIM], m[DIM], A[NE];
   load_pt<DIM>(pos0, i, p);
+  CellBounds<DIM, TESS> bounds;
+  const uint64_t all = __builtin_amdgcn_read_exec();
+  uint64_t in = 0;  // lanes whose point is in the cell of their row
   for (int s = 0; s < nSteps; s++) {
-    const double* A = Atab + cell_of<DIM, TESS, POW2>(p, g) * NE;
+    if (in != all) {
+      const int c = cell_of<DIM, TESS, POW2>(p, g);
+#pragma unroll
+      for (int e = 0; e < NE; e++) A[e] = Atab[c * NE + e];
+      bounds.enter(p, c, g);
+    }
     affine<DIM>(y, A, p);
 #pragma unroll
-    for (int d = 0; d < DIM; d++) m[d] = p[d] + h * y[d] / 2.;
+    for (int d = 0; d < DIM; d++) m[d] = p[d] + hh * y[d];
     affine<DIM>(y, A, m);
 #pragma unroll
     for (int d = 0; d < DIM; d++) p[d] += y[d] * h;
+    in = bounds.inside(p, g);
   }
   store_pt<DIM>(out, i, p);
 }
