@@ -40,8 +40,9 @@
 // pass, its accepted ones ~50 a step), and below ~20 pairs of 128 x 128
 // pixels the corner's pixel alone, one chain of nT nS substeps.  64 pairs of
 // 128 x 128, 100 steps, 10 substeps: 1.72 ms with a checkpoint, a lookup and
-// a dependent load for every step, 1.03 with events, 0.69 with the last lane's
-// events spread (4 pairs: 0.97, 0.97 and 0.46).
+// a dependent load for every step, 1.03 with events, 0.68 with the last lane's
+// events spread (4 pairs: 0.97, 0.97 and 0.46; 0.39 with the corner's own
+// forward loop, corner_steps).
 //
 // Accumulation, bit-reproducible: each lane keeps two register
 // accumulators, dJ/dA of its current RK2 cell and dJ/dTrel of its current
@@ -269,6 +270,25 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
         const uint64_t todo = ballot(t < nT);
         if (todo == 0) break;
         bool waits = t < nT;
+        if (TESS == TESS_I && POW2 && cool > 0 && __popcll(todo) == 1) {  // one lane left, and no stretch for it
+          if (waits && (c == 0 || c == 3) && __builtin_fabs(p[0]) < 0.125 * g.inc_x &&
+              __builtin_fabs(p[1]) < 0.125 * g.inc_y) {
+            corner_steps(
+                p, c, t, nT, Tr, At, h, nS, g,
+                [&](int c0, int c1) {
+                  if (has_sig) sg = sig_mix(sig_mix(sg, c0), c1);
+                },
+                [&](int c0) {
+                  if (has_sig) sg = sig_mix(sg, c0);
+                },
+                [&](int, int c0, bool redo, const double* q, const double*) {
+                  log_start(q);
+                  log_event(c0, redo ? 0 : 1);
+                  nredo += redo ? 1 : 0;
+                });
+            waits = false;
+          }
+        }
         if (cool > 0) {
           cool--;
         } else {

@@ -464,16 +464,23 @@ constexpr int kRefill = 8;
 // substep, so up to all its steps are redone, one dependent chain of 1 100
 // units where its neighbours have ~110, and the wave (a launch of 512 x 512
 // grid points: all of it) waits for it.  Alone in its wave it runs here to
-// step tb: the two triangles' rows stay in registers, a branch picks one, and
-// the lookup is two products and three comparisons while the point is within
-// an eighth of a box of the corner, where the reference's rules
-// (calc_2Dto2D.cu:60-110) come down to: left of the corner (px <= 0) triangle
-// 3 unless sy < sx, else 3 where sx < sy and 0 elsewhere (1 - x < y holds for
-// no point this near).  Returns where it has left that neighbourhood.
-template <int MODE>
-__device__ __forceinline__ void corner_steps(double* p, int& c, int& t, int tb, int& nfb, const double* Ttab,
-                                             const double* Atab, double h, int nS, const Geom& g,
-                                             double* __restrict__ traj, int64_t nPts) {
+// step tb: the two triangles' rows stay in registers, and the lookup is a few
+// products and comparisons while the point is within an eighth of a box of
+// the corner, where the reference's rules (calc_2Dto2D.cu:60-110) come down
+// to: left of the corner (px <= 0) triangle 3 unless sy < sx, else 3 where
+// sx < sy and 0 elsewhere (1 - x < y holds for no point this near).  So 3
+// where sx < sy and 0 where sy < sx: the substeps' loop asks no more and
+// leaves a tie or a point further out to `cell`.  It is one dependent chain
+// of a lone wave, ~270 cycles a substep (570 with the whole rule and
+// a branch per triangle in it): a 512 x 512 grid with a flipping corner 264 ->
+// 195 us, the adjoint of 16 pairs of 128 x 128 (its forward sweep) 490 -> 380.
+// Returns where it has left that neighbourhood.
+// The caller's hooks: proposed(cell, cell of the proposal), substep(cell it
+// starts in), done(step, cell, redone, start point, end point).
+template <class Proposed, class Substep, class Done>
+__device__ __forceinline__ void corner_steps(double* p, int& c, int& t, int tb, const double* Ttab,
+                                             const double* Atab, double h, int nS, const Geom& g, Proposed proposed,
+                                             Substep on_substep, Done done) {
   const double hh = h * 0.5, mx = 0.125 * g.inc_x, my = 0.125 * g.inc_y;
   double A0[6], A3[6];
 #pragma unroll
@@ -504,22 +511,40 @@ __device__ __forceinline__ void corner_steps(double* p, int& c, int& t, int tb, 
   const int te = __builtin_amdgcn_readfirstlane(tb);
   int tu = __builtin_amdgcn_readfirstlane(t);
   while (near && tu < te) {
+    const double q[2] = {p[0], p[1]};
+    const int cq = cu;
     double y[2];
     affine<2>(y, Ttab + cu * 6, p);
     const int cy = cell(y, near);
-    if (cy == cu) {
+    proposed(cu, cy);
+    const bool redo = cy != cu;
+    if (!redo) {
       p[0] = y[0];
       p[1] = y[1];
     } else {
-      nfb++;
-      for (int s = 0; s < nS; s++) {
-        if (cu == 0) substep(A0);
-        else if (cu == 3) substep(A3);
-        else substep(Atab + cu * 6);
-        cu = cell(p, near);
+      near = true;
+      int s = nS;
+      while (s > 0 && near) {
+        uint64_t plain;  // beyond doubt: within a sixteenth of a box and on one side
+        do {
+          on_substep(cu);
+          if (cu == 3) substep(A3);
+          else substep(A0);
+          const double sx = p[0] * g.rinc_x, sy = p[1] * g.rinc_y;
+          const uint64_t lt = lanes_lt(sx, sy);
+          plain = (lt | lanes_lt(sy, sx)) & lanes_lt(__builtin_fmax(__builtin_fabs(sx), __builtin_fabs(sy)), 0.0625);
+          cu = lt != 0 ? 3 : 0;
+          s--;
+        } while (s > 0 && plain != 0);
+        if (plain == 0) cu = cell(p, near);
+      }
+      for (; s > 0; s--) {  // (it has left: the step's other substeps)
+        on_substep(cu);
+        substep(Atab + cu * 6);
+        cu = __builtin_amdgcn_readfirstlane(cell2<TESS_I, true>(p, g));
       }
     }
-    if (MODE == 1) store_pt<2>(traj, (int64_t)tu * nPts, p);
+    done(tu, cq, redo, q, p);
     tu++;
   }
   c = cu;
@@ -549,7 +574,12 @@ __device__ __forceinline__ void advance(double* p, int& c, int& t, int tb, int& 
     if (DIM == 2 && TESS == TESS_I && POW2 && nTodo == 1 && cool > 0) {  // one lane left, and no stretch for it
       if (waits && (c == 0 || c == 3) && __builtin_fabs(p[0]) < 0.125 * g.inc_x &&
           __builtin_fabs(p[1]) < 0.125 * g.inc_y) {
-        corner_steps<MODE>(p, c, t, tb, nfb, Ttab, Atab, h, nS, g, traj, nPts);
+        corner_steps(
+            p, c, t, tb, Ttab, Atab, h, nS, g, [](int, int) {}, [](int) {},
+            [&](int step, int, bool redo, const double*, const double* q) {
+              nfb += redo ? 1 : 0;
+              if (MODE == 1) store_pt<2>(traj, (int64_t)step * nPts, q);
+            });
         waits = false;
       }
     }

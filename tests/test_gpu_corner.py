@@ -1,0 +1,54 @@
+"""calc_T of a lone point beside the domain's corner.
+
+There it runs in a loop of its own while it stays within an eighth of a box
+(within a sixteenth without ties by a shorter rule).  The points lie on the
+diagonal between the corner box's triangles 0 and 3 and its extension, around
+those distances, on it up to rounding, and on the walls; fields either vanish
+across the walls or carry the points out of the neighbourhood within a step.
+End points, fallback counts, trajectories and the adjoint's end points must
+equal the oracle's bit for bit (cpab/gpu/calc_2Dto2D.cu:60-110, 348-408)."""
+import numpy as np
+import pytest
+
+from cpabdiffeo_amd import adjoint
+from cpabdiffeo_amd.calcs import Calcs
+from cpabdiffeo_amd.space import CpaSpace
+
+pytestmark = pytest.mark.gpu
+
+AT = [0.0, 1e-300, 1e-17, 1e-3, 0.0624, 0.0625, 0.0626, 0.12499, 0.125, 0.13]
+
+
+@pytest.mark.parametrize("zero,speed", [(True, 1.0), (False, 0.02), (False, 1.0)])
+@pytest.mark.parametrize("nCs,extent", [((4, 4), (1.0, 1.0)), ((2, 2), (64.0, 32.0))])
+def test_lone_points_equal_the_oracle(gpu, orc, nCs, extent, zero, speed):
+    torch = gpu
+    print("[gpu] corner", nCs, extent, zero, speed, flush=True)
+    sp = CpaSpace([0, 0], list(extent), list(nCs), zero_v_across_bdry=[zero] * 2, tess="I", valid_outside=not zero)
+    inc = np.array(extent) / np.array(nCs)
+    pts = np.array([(s * a * f, t * a) for a in AT for s, t in [(1, 1), (-1, -1), (1, 0), (0, 1), (1, -1), (-1, 1)]
+                    for f in (1.0, 1.0 + 2e-16, 1.0 - 1.2e-16)]) * inc
+    g, dt, nT, nS = sp.tessellation.geom(), 0.05, 20, 10
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()  # noqa: E731
+    calcs = Calcs(sp.nC, np.float64, 2, 2, "I")
+    for seed in range(3):
+        A = (sp.B @ np.random.default_rng(seed).normal(size=sp.d)).reshape(sp.nC, 2, 3)
+        A *= speed / max(np.abs(A[:, :, :2]).max(), np.abs(A[:, :, 2] / np.array(extent)).max())
+        sA, T = orc.prep(2, A.reshape(sp.nC, 6), 1, dt)
+        want, nfb_w, _ = orc.calc_T(g, pts, T, sA, dt, nT, nS, probe=True)
+        traj_w = orc.calc_trajectory(g, pts, T, sA, dt, nT, nS)
+        dT, dA, dp = dev(T.reshape(sp.nC, 6)), dev(sA.reshape(sp.nC, 6)), dev(pts)
+        out, pos = torch.zeros_like(dp), torch.zeros_like(dp)
+        nfb = torch.zeros(len(pts), dtype=torch.int32, device="cuda")
+        traj = torch.zeros((nT, len(pts), 2), dtype=torch.float64, device="cuda")
+        lam = torch.ones((1, 2), dtype=torch.float64, device="cuda")
+        for i in range(len(pts)):
+            calcs.calc_T(None, None, dT, dA, dp[i:i + 1], dt, nT, nS, out[i:i + 1], 2, 2, sp.nCs, sp.incs,
+                         n_fallback=nfb[i:i + 1])
+            traj[:, i] = calcs.calc_trajectory(None, None, dT, dA, dp[i:i + 1], dt, nT, nS, 2, 2, sp.nCs, sp.incs)[:, 0]
+            adjoint.calc_T_vjp(sp, dp[i:i + 1], lam, dA, dT, dict(dt=dt, nTimeSteps=nT, nStepsODEsolver=nS),
+                               pos_out=pos[i:i + 1])
+        assert np.array_equal(out.cpu().numpy(), want)
+        assert np.array_equal(pos.cpu().numpy(), want)
+        assert np.array_equal(nfb.cpu().numpy(), nfb_w)
+        assert np.array_equal(traj.cpu().numpy(), traj_w)
