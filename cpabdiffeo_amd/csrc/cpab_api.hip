@@ -222,7 +222,8 @@ int launch_integrate_t(cpab_ctx* ctx, int mode, const Shape& s, const double* po
   if (mode == 0) {
     auto k = k_integrate<DIM, TESS, POW2, LDS, 0>;
     allow_lds(k, s.lds);
-    hipLaunchKernelGGL(k, dim3((unsigned)s.grid), dim3(s.block), s.lds, ctx->stream, pos0, out, Trels, As, h, nT, nS,
+    const int64_t blocks = s.grid + (has_corner_block(DIM, TESS, POW2, 0) ? 1 : 0);
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(s.block), s.lds, ctx->stream, pos0, out, Trels, As, h, nT, nS,
                        nPts, g, nC, s.ptsPerWave, nfb, ps);
   } else {
     auto k = k_integrate<DIM, TESS, POW2, LDS, 1>;

@@ -710,12 +710,19 @@ __device__ __forceinline__ GridOrder grid_order(int w, int64_t n) {
 // with a range for each wave the block waited for the one whose points cross
 // the most facets (256 batched instances, 16 waves a block: 11.4 -> 9.6 ms).
 // Block-uniform arguments; every lane of the block calls it.
+//
+// corner: a grid that starts beside the domain's corner has its first point
+// integrated by a block of its own (2), and the block that it falls to leaves
+// it out (1): it may be `corner_steps`'s, and among 63 neighbours it took one
+// step to their stretch of 32 until they were done (512 x 512 grid with a
+// flipping corner 195 -> 163 us; other launches, one block more, the same).
 template <int DIM, int TESS, bool POW2, int MODE>
 __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* cursor, const double* __restrict__ pos0,
                                                 double* __restrict__ out, const double* Ttab, const double* Atab,
                                                 double h, int nT, int nS, int64_t nPts, const Geom& g,
                                                 int32_t* __restrict__ nfb_out, const GridOrder& gord = GridOrder(),
-                                                int64_t gbase = 0, const uint16_t* lord = nullptr) {
+                                                int64_t gbase = 0, const uint16_t* lord = nullptr,
+                                                int corner = 0) {
   // a grid's tiles are 64 neighbouring points that need similar work, so a
   // wave takes one after another (2048 x 2048 points: 750 -> 610 us); other
   // waves take the next points as soon as kRefill lanes are free (256 batched
@@ -725,6 +732,22 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* curso
   int c = 0, t = 0, nfb = 0;
   int64_t my = 0;
   bool active = false, more = true;
+  int taken = 0;  // points the cursor leaves out
+  if (DIM == 2 && TESS == TESS_I && POW2 && MODE == 0 && corner != 0) {
+    bool near = false;
+    if (gord.w > 0) {
+      my = gbase + gord(begin - gbase);
+      load_pt<DIM>(pos0, my, p);
+      near = ballot(__builtin_fabs(p[0]) < 0.125 * g.inc_x && __builtin_fabs(p[1]) < 0.125 * g.inc_y) != 0;
+    }
+    if (corner == 2) {
+      if (!near) return;
+      active = threadIdx.x == 0;
+      more = false;
+      c = cell_of<DIM, TESS, POW2>(p, g);
+    }
+    taken = near ? 1 : 0;
+  }
   for (;;) {
     if (active && t >= nT) {  // retire a finished point
       if (MODE == 0) store_pt<DIM>(out, my, p);
@@ -737,7 +760,7 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* curso
       if (lane_id() == 0) next = atomicAdd(cursor, __popcll(idle));
       next = __builtin_amdgcn_readfirstlane(next);
       if (!active) {
-        const int cand = next + rank_in(idle);
+        const int cand = next + taken + rank_in(idle);
         if (cand < n) {
           my = gord.w > 0 ? gbase + gord(begin - gbase + cand) : begin + (lord ? (int)lord[cand] : cand);
           active = true;
@@ -747,13 +770,19 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* curso
           nfb = 0;
         }
       }
-      more = next + __popcll(idle) < n;
+      more = next + taken + __popcll(idle) < n;
     }
     if (ballot(active) == 0) break;
     if (!active || t >= nT) continue;
     advance<DIM, TESS, POW2, MODE>(p, c, t, nT, nfb, Ttab, Atab, h, nS, g, more, refill,
                                    MODE == 1 ? out + my * DIM : nullptr, nPts);
   }
+}
+
+// Launches of k_integrate that have a block ahead of the points' own, for the
+// corner's point (the cases of `corner_steps`).
+constexpr bool has_corner_block(int dim, int tess, bool pow2, int mode) {
+  return mode == 0 && dim == 2 && tess == TESS_I && pow2;
 }
 
 template <int DIM, int TESS, bool POW2, bool LDS, int MODE>
@@ -766,6 +795,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5)))
   extern __shared__ double lds[];
   __shared__ int grid_w, cursor;
   constexpr bool kDetect = MODE == 0 && DIM > 1;
+  constexpr bool kCorner = has_corner_block(DIM, TESS, POW2, MODE);  // block 0 is the corner's
   RowProbe<DIM> probe;
   if (threadIdx.x == 0) {
     grid_w = 0x7fffffff;
@@ -788,9 +818,11 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5)))
     gord = grid_order(grid_w, nPts);
   }
   const int per = (int)(blockDim.x >> 6) * ptsPerWave;
-  const int64_t begin = (int64_t)blockIdx.x * per;
+  const int64_t blk = kCorner ? (blockIdx.x == 0 ? 0 : (int64_t)blockIdx.x - 1) : (int64_t)blockIdx.x;
+  const int64_t begin = blk * per;
   const int n = nPts - begin < per ? (int)(nPts - begin) : per;
-  integrate_range<DIM, TESS, POW2, MODE>(begin, n, &cursor, pos0, out, Ttab, Atab, h, nT, nS, nPts, g, nfb_out, gord);
+  integrate_range<DIM, TESS, POW2, MODE>(begin, n, &cursor, pos0, out, Ttab, Atab, h, nT, nS, nPts, g, nfb_out, gord, 0,
+                                         nullptr, !kCorner ? 0 : blockIdx.x == 0 ? 2 : blockIdx.x == 1 ? 1 : 0);
 }
 
 // ---------------------------------------------------------- sensitivity

@@ -52,3 +52,27 @@ def test_lone_points_equal_the_oracle(gpu, orc, nCs, extent, zero, speed):
         assert np.array_equal(pos.cpu().numpy(), want)
         assert np.array_equal(nfb.cpu().numpy(), nfb_w)
         assert np.array_equal(traj.cpu().numpy(), traj_w)
+
+
+@pytest.mark.parametrize("rows,cols", [(8, 64), (16, 8), (64, 64), (129, 72), (40, 65), (512, 64)])
+@pytest.mark.parametrize("offset", [0.0, -1e-17, 0.03, 0.2])
+def test_grids_from_the_corner_equal_the_oracle(gpu, orc, rows, cols, offset):
+    """A grid's first point beside the corner is integrated by a block of its own."""
+    torch = gpu
+    print("[gpu] corner grid", rows, cols, offset, flush=True)
+    sp = CpaSpace([0, 0], [1, 1], [4, 4], zero_v_across_bdry=[True] * 2, tess="I")
+    y, x = np.mgrid[0:rows, 0:cols]
+    pts = np.stack([x.ravel() / cols, y.ravel() / rows], 1) * 0.9 + offset
+    g, dt, nT, nS = sp.tessellation.geom(), 0.05, 20, 10
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    calcs = Calcs(sp.nC, np.float64, 2, 2, "I")
+    for seed in range(4):
+        A = (sp.B @ np.random.default_rng(seed).normal(size=sp.d)).reshape(sp.nC, 6)
+        sA, T = orc.prep(2, A / np.abs(A).max(), 1 - 2 * (seed & 1), dt)
+        want, nfb_w, _ = orc.calc_T(g, pts, T, sA, dt, nT, nS, probe=True)
+        out = torch.zeros(pts.shape, dtype=torch.float64, device="cuda")
+        nfb = torch.full((len(pts),), -1, dtype=torch.int32, device="cuda")
+        calcs.calc_T(None, None, dev(T.reshape(sp.nC, 6)), dev(sA.reshape(sp.nC, 6)), dev(pts), dt, nT, nS, out, 2, 2,
+                     sp.nCs, sp.incs, n_fallback=nfb)
+        assert np.array_equal(out.cpu().numpy(), want)
+        assert np.array_equal(nfb.cpu().numpy(), nfb_w)
