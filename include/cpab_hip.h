@@ -215,7 +215,8 @@ typedef struct {
 } cpab_batch_inst;
 
 /* Schedule of the persistent launch: points per tile, threads per block
- * (a multiple of 64, at most 1024), tiles a block takes per queue grab. */
+ * (a multiple of 64, at most 1024), tiles a block takes per queue grab (a
+ * batch takes fewer towards its end, work items more while many wait). */
 typedef struct {
   int tile;
   int block;
