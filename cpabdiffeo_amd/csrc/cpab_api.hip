@@ -522,7 +522,8 @@ int cpab_calc_grad_theta(cpab_ctx* ctx, int dim, int tess, int nC, const double*
   const int64_t waves = (nPts + 63) / 64;
   int jc = dim == 3 ? 4 : 8;
   while (jc > 1 && waves * ((d + jc - 1) / jc) < 3 * (int64_t)ctx->n_cu) jc >>= 1;
-  const dim3 grid((unsigned)((nPts + 255) / 256), (unsigned)((d + jc - 1) / jc));
+  const unsigned chunks = (unsigned)((d - 1) / jc + 1), cy = chunks < 32768u ? chunks : 32768u;
+  const dim3 grid((unsigned)((nPts + 255) / 256), cy, (chunks + cy - 1) / cy);
 #define GRAD_RUN(J_)                                                                                         \
   hipLaunchKernelGGL((k_grad_theta<D_, T_, P_, J_>), grid, dim3(256), 0, ctx->stream, pos0, pos, As, Bs, grad, \
                      d, h, (int)steps64, nPts, g, nC)

@@ -851,7 +851,9 @@ __global__ void __launch_bounds__(256, 2)
                  const double* __restrict__ Bs, double* __restrict__ grad, int d, double h, int nSteps,
                  int64_t nPts, Geom g, int nC) {
   constexpr int NE = DIM * (DIM + 1);
-  const int jc = (int)blockIdx.y * JC, j0 = jc + JC <= d ? jc : (d > JC ? d - JC : 0);
+  const int64_t jc = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * JC;
+  if (jc >= d) return;
+  const int j0 = jc + JC <= d ? (int)jc : (d > JC ? d - JC : 0);
   const int nj = d < JC ? d : JC;
   const double* Bl = Bs + (int64_t)j0 * nC * NE;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -904,7 +906,7 @@ __global__ void __launch_bounds__(256, 2)
     for (int i = 0; i < DIM; i++) p[i] += v[i] * h;
     in = bounds.inside(p, g);
   }
-  if (blockIdx.y == 0) store_pt<DIM>(pos, idx, p);
+  if (jc == 0) store_pt<DIM>(pos, idx, p);
 #pragma unroll
   for (int jj = 0; jj < JC; jj++)
     if (jj < nj)
