@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
           double R[6];
 #pragma unroll
           for (int e = 0; e < 6; e++) R[e] = Tr[c * 6 + e];
-          B.enter(p, c, g);
+          B.enter(c, g);
           uint64_t go = B.inside(p, g) & todo;
           if (go == 0) cool = 8;
           for (int s = 0; s < kAdjSegs && go != 0; s++) {

@@ -135,6 +135,8 @@ int make_geom(cpab_ctx* ctx, int dim, int tess, int nC0, int nC1, int nC2, doubl
   g->eps = (nmax + 16.0) * 0x1p-46 + 2e-10 * rmax;
   g->sc1 = 1.0 / (1.0 - 2.0 * g->eps);
   g->sc17 = 1.0 / (17.0 - g->eps);
+  g->rn0 = 1.0 / (double)nC0;
+  g->rn01 = 1.0 / ((double)nC0 * (double)nC1);
   // The type I clamps must leave a non-empty range, or the box index of a
   // clamped point would be negative.
   if (tess == TESS_I && !(g->top_x > 0.0 && g->top_y > 0.0 && (dim < 3 || g->top_z > 0.0)))

@@ -34,11 +34,12 @@ constexpr int TESS_II = 2;  // intervals / rectangles / boxes (TESS_TYPE 2)
 struct Geom {
   int nC0, nC1, nC2, pad;
   double inc_x, inc_y, inc_z;
-  double rinc_x, rinc_y, rinc_z;  // exact 1/inc (POW2 form only)
+  double rinc_x, rinc_y, rinc_z;  // 1 / inc: exact for powers of two, else rounded
   double top_x, top_y, top_z;     // clamps nC0*inc_x-1e-10, nC1*inc_y-1e-10, nC2*inc_x-1e-10
   double wall_x, wall_y;          // nC0*inc_x, nC1*inc_y (2D type I out-of-domain tests)
   double eps;                     // margin of CellBounds, in increments
   double sc1, sc17;               // 1 / (1 - 2 eps), 1 / (17 - eps): its scales (2D type I)
+  double rn0, rn01;               // 1 / nC0, 1 / (nC0 nC1) (box_of)
 };
 
 __device__ __forceinline__ double dmin(double a, double b) { return __builtin_fmin(a, b); }
@@ -306,6 +307,24 @@ __device__ __forceinline__ int cell_of(const double* p, const Geom& g) {
   if (DIM == 1) return cell1<POW2>(p, g);
   if (DIM == 2) return cell2<TESS, POW2, FAST, EARLY>(p, g);
   return cell3<TESS, POW2>(p, g);
+}
+
+// The box with index b: its place along each axis, as doubles.  b + 1/2 is at
+// least half a count from a multiple of n, so the products' rounding (b < 2^24)
+// never changes the floors.
+template <int DIM>
+__device__ __forceinline__ void box_of(int b, const Geom& g, double* k) {
+  double r = (double)b;
+  if (DIM == 3) {
+    const double n01 = (double)mul24(g.nC0, g.nC1);
+    k[2] = __builtin_floor((r + 0.5) * g.rn01);
+    r = __builtin_fma(-n01, k[2], r);
+  }
+  if (DIM >= 2) {
+    k[1] = __builtin_floor((r + 0.5) * g.rn0);
+    r = __builtin_fma(-(double)g.nC0, k[1], r);
+  }
+  k[0] = r;
 }
 
 // ------------------------------------------------------ affine products

@@ -285,27 +285,30 @@ __device__ __forceinline__ uint64_t lanes_ge(double a, double b) { return __buil
 __device__ __forceinline__ uint64_t lanes_lt(int a, int b) { return __builtin_amdgcn_sicmp(a, b, 40); }
 __device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
 
-// Whether points that came from their cells c are still in them, without a
-// lookup: a few affine functions of the point against bounds set once for the
-// cell.  The bounds lie g.eps inside the cell (the roundings of this test and
-// of the lookup's own arithmetic, and the lookup's clamp 1e-10 inside the far
-// walls), so a lane of inside(q) is one whose lookup of q gives c; one that is
-// turned down is looked up.  NaN and infinite points are turned down.
+// Whether points are in their cells c, without a lookup: a few affine
+// functions of the point against bounds set once for the cell.  The bounds lie
+// g.eps inside the cell (the roundings of this test and of the lookup's own
+// arithmetic, and the lookup's clamp 1e-10 inside the far walls), so a lane of
+// inside(q) is one whose lookup of q gives c; one that is turned down is looked
+// up.  NaN and infinite points are turned down.  The box is c's own, from its
+// index: one found again from the point can be c's neighbour (a point just
+// below a multiple of the increment rounds up in p * (1 / inc)), and a row kept
+// within a neighbour's bounds is the wrong one from there on.
 //
 // Boxes (1D, type II): a lower and an upper bound per axis, none on the sides
 // of the domain (the lookup clamps, so what lies beyond belongs to the box).
 template <int DIM, int TESS>
 struct CellBounds {
   double lo[DIM], hi[DIM];
-  __device__ __forceinline__ void enter(const double* p, int, const Geom& g) {
+  __device__ __forceinline__ void enter(int c, const Geom& g) {
     const int nC[3] = {g.nC0, g.nC1, g.nC2};
-    const double inc[3] = {g.inc_x, g.inc_y, g.inc_z}, rinc[3] = {g.rinc_x, g.rinc_y, g.rinc_z};
+    const double inc[3] = {g.inc_x, g.inc_y, g.inc_z};
+    double k[DIM];
+    box_of<DIM>(c, g, k);
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
-      const double n1 = (double)(nC[d] - 1);
-      const double k = dmin(n1, dmax(0.0, __builtin_floor(p[d] * rinc[d])));
-      lo[d] = k > 0.0 ? (k + g.eps) * inc[d] : -__DBL_MAX__;
-      hi[d] = k < n1 ? (k + 1.0 - g.eps) * inc[d] : __DBL_MAX__;
+      lo[d] = k[d] > 0.0 ? (k[d] + g.eps) * inc[d] : -__DBL_MAX__;
+      hi[d] = k[d] < (double)(nC[d] - 1) ? (k[d] + 1.0 - g.eps) * inc[d] : __DBL_MAX__;
     }
   }
   __device__ __forceinline__ uint64_t inside(const double* q, const Geom&) const {
@@ -329,10 +332,11 @@ template <>
 struct CellBounds<2, TESS_I> {
   double k1, k2, ax, by, mid;
   uint64_t above1, above2;  // lanes whose u lies at or above k1, whose v above k2
-  __device__ __forceinline__ void enter(const double* p, int c, const Geom& g) {
+  __device__ __forceinline__ void enter(int c, const Geom& g) {
     const double ni = (double)(g.nC0 - 1), nj = (double)(g.nC1 - 1);
-    const double i = dmin(ni, dmax(0.0, __builtin_floor(p[0] * g.rinc_x)));
-    const double j = dmin(nj, dmax(0.0, __builtin_floor(p[1] * g.rinc_y)));
+    double box[2];
+    box_of<2>(c >> 2, g, box);
+    const double i = box[0], j = box[1];
     // c & 3: 0 top, 1 right, 2 bottom, 3 left
     const bool b1 = (c & 2) != 0;        // sx - i < sy - j
     const bool b2 = ((c + 1) & 2) != 0;  // their sum > 1
@@ -375,16 +379,13 @@ template <>
 struct CellBounds<3, TESS_I> {
   double k1, k2, k3, k4, fx, fy, fz, zmax;
   uint64_t a1, a2, a3, a4, lx, ly, lz;  // lanes above the planes, lanes whose side is the lower one
-  __device__ __forceinline__ void enter(const double* p, int c, const Geom& g) {
-    const double ni = (double)(g.nC0 - 1), nj = (double)(g.nC1 - 1), nk = (double)(g.nC2 - 1);
-    const double i = dmin(ni, dmax(0.0, __builtin_floor(p[0] * g.rinc_x)));
-    const double j = dmin(nj, dmax(0.0, __builtin_floor(p[1] * g.rinc_y)));
-    const double k = dmin(nk, dmax(0.0, __builtin_floor(p[2] * g.rinc_z)));
-    const int ii = (int)i, ij = (int)j, ik = (int)k;
-    // (another box than c's, next to a side, leaves 0 .. 4 and lies within no bounds)
-    const int tet = c - mul24(ii + mul24(ij, g.nC0) + mul24(ik, mul24(g.nC1, g.nC0)), 5);
-    const bool ok = (unsigned)tet < 5u;
-    const bool tf = ((ii + ij + ik) & 1) != 0;
+  __device__ __forceinline__ void enter(int c, const Geom& g) {
+    const double ni = (double)(g.nC0 - 1), nj = (double)(g.nC1 - 1);
+    const int b = (int)(((double)c + 0.5) * 0.2), tet = c - mul24(b, 5);  // (a tenth or more from rounding up)
+    double box[3];
+    box_of<3>(b, g, box);
+    const double i = box[0], j = box[1], k = box[2];
+    const bool tf = (((int)i + (int)j + (int)k) & 1) != 0;
     const bool t1 = tet == 1, t2 = tet == 2, t3 = tet == 3, t4 = tet == 4;
     const bool b1 = tf ? !t4 : t1, b2 = tf ? !t3 : t2, b3 = tf ? t1 : !t3, b4 = tf ? t2 : !t4;
     const double e = 4.0 * g.eps;
@@ -405,8 +406,7 @@ struct CellBounds<3, TESS_I> {
     lx = ballot(!ux);
     ly = ballot(!uy);
     lz = ballot(!uz);
-    const double wall = dmin(((double)g.nC2 - e) * g.inc_z, g.top_z - e * g.inc_z);
-    zmax = ok ? wall : -__DBL_MAX__;
+    zmax = dmin(((double)g.nC2 - e) * g.inc_z, g.top_z - e * g.inc_z);
   }
   __device__ __forceinline__ uint64_t inside(const double* q, const Geom& g) const {
     const double ty = q[1] * g.rinc_y;
@@ -591,7 +591,7 @@ __device__ __forceinline__ void advance(double* p, int& c, int& t, int tb, int& 
       const double* row = Ttab + mul24(c, NE);
 #pragma unroll
       for (int e = 0; e < NE; e++) R[e] = row[e];
-      B.enter(p, c, g);
+      B.enter(c, g);
       uint64_t go = B.inside(p, g) & todo;  // the lanes of the stretch
       if (go == 0) cool = 8;
       for (;;) {
@@ -883,7 +883,7 @@ __global__ void __launch_bounds__(256, 2)
             for (int e = 0; e < NE; e++) B[jj][e] = Bl[((jj < nj ? jj : 0) * nC + c) * NE + e];
         }
       }
-      bounds.enter(p, c, g);
+      bounds.enter(c, g);
     }
     double v[DIM], pMid[DIM];
     affine<DIM>(v, A, p);
@@ -945,7 +945,7 @@ __global__ void __launch_bounds__(1024)
       const int c = cell_of<DIM, TESS, POW2>(p, g);
 #pragma unroll
       for (int e = 0; e < NE; e++) A[e] = Atab[c * NE + e];
-      bounds.enter(p, c, g);
+      bounds.enter(c, g);
     }
     affine<DIM>(y, A, p);
 #pragma unroll
