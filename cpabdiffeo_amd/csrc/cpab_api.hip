@@ -1030,6 +1030,7 @@ int cpab_batch_calc_T(cpab_batch* b, const double* tables, const double* pos0, d
   cpab_batch_sched q = sched ? *sched : cpab_batch_sched{16384, 1024, 4};
   if (q.tile < 64 || q.block < 64 || q.block > 1024 || (q.block & 63) || q.chunk < 1)
     return fail(ctx, CPAB_ERR_ARG, "schedule: tile >= 64, block a multiple of 64 up to 1024, chunk >= 1");
+  if (q.tile > kItemMax) q.tile = kItemMax;
   if (nT < 0 || nS < 0) return fail(ctx, CPAB_ERR_ARG, "negative step counts");
   if (b->nPts == 0) return CPAB_OK;
   if (!tables || !pos0 || !out) return fail(ctx, CPAB_ERR_ARG, "null pointer argument");

@@ -75,7 +75,11 @@ __global__ void k_batch_reset(unsigned int* queue) {
 // when, never the point's result.
 constexpr int kBucketTileMax = 16384;  // the most points of a sorted tile (16-bit indices)
 constexpr int kBucketMax = 1024;       // buckets
-constexpr int kItemMax = 1 << 30;      // the most points of an item taken at a time (32-bit cursor)
+// The most points of a tile or an item taken at a time: a block's waves draw
+// them from a 32-bit cursor, which each wave's last draw leaves up to 64 past
+// the end (integrate_range's `next + taken + 64` is the largest sum).
+constexpr int kItemMax = 1 << 30;
+static_assert((int64_t)kItemMax + 64 * (1024 / 64) + 1 + 64 <= INT32_MAX, "integrate_range's cursor");
 
 template <int DIM>
 __device__ __forceinline__ int bucket_of(const double* p, const double* sc, int nb) {

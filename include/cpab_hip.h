@@ -214,8 +214,8 @@ typedef struct {
   int64_t nPts;
 } cpab_batch_inst;
 
-/* Schedule of the persistent launch: points per tile, threads per block
- * (a multiple of 64, at most 1024), tiles a block takes per queue grab (a
+/* Schedule of the persistent launch: points per tile (a batch takes at most
+ * 2^30), threads per block (a multiple of 64, at most 1024), tiles a block takes per queue grab (a
  * batch takes fewer towards its end, work items more while many wait). */
 typedef struct {
   int tile;
