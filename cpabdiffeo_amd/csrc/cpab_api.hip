@@ -175,7 +175,7 @@ struct Shape {
 Shape integrate_shape(const cpab_ctx* ctx, int64_t nPts, int nC, int ne, int ntables) {
   Shape s;
   const size_t tbytes = (size_t)ntables * nC * ne * sizeof(double);
-  s.use_lds = tbytes <= (size_t)ctx->max_lds;
+  s.use_lds = tbytes + kOwnLds <= (size_t)ctx->max_lds;
   s.lds = s.use_lds ? tbytes : 0;
   s.block = (s.lds > 32768) ? 1024 : 256;
   // waves wanted: 8 per SIMD (4 SIMDs per CU); each lane takes ceil of the rest
@@ -890,7 +890,7 @@ int batch_launch(cpab_batch* b, hipStream_t s, const cpab_batch_sched& q, const 
   // uniform random points, tiles of 16 384: 54.4 -> 43.9 ms)
   int sort_off = 0;
   const size_t lds_sorted = lds + sizeof(unsigned int) * kBucketMax + sizeof(uint16_t) * (size_t)q.tile;
-  if (q.tile <= kBucketTileMax && lds_sorted <= (size_t)ctx->max_lds) {
+  if (q.tile <= kBucketTileMax && lds_sorted + kOwnLds <= (size_t)ctx->max_lds) {
     sort_off = 2 * b->maxNC * NE;
     lds = lds_sorted;
   }
@@ -1100,7 +1100,7 @@ int items_launch(cpab_ctx* ctx, const WorkItem* items, unsigned int* queue, int 
   if (DIM == 1 && maxLen <= kBucketTileMax) {
     sort_cap = maxLen * kGrabMax < kBucketTileMax ? (int)maxLen * kGrabMax : kBucketTileMax;
     const size_t lds_sorted = lds + sizeof(unsigned int) * kBucketMax + sizeof(uint16_t) * (size_t)sort_cap;
-    if (lds_sorted <= (size_t)ctx->max_lds) {
+    if (lds_sorted + kOwnLds <= (size_t)ctx->max_lds) {
       sort_off = 2 * maxNC * NE;
       lds = lds_sorted;
     }

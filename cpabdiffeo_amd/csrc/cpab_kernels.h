@@ -785,6 +785,10 @@ constexpr bool has_corner_block(int dim, int tess, bool pow2, int mode) {
   return mode == 0 && dim == 2 && tess == TESS_I && pow2;
 }
 
+// LDS that the integration kernels hold besides their tables and orders (the
+// cursors, a run's row length): a launch's dynamic LDS leaves room for it.
+constexpr int kOwnLds = 16;
+
 template <int DIM, int TESS, bool POW2, bool LDS, int MODE>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5)))
     k_integrate(const double* __restrict__ pos0, double* __restrict__ out,
