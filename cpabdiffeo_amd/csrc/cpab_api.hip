@@ -1095,7 +1095,11 @@ int items_launch(cpab_ctx* ctx, const WorkItem* items, unsigned int* queue, int 
   // built in LDS after the tables (tile_bucket_order).  Measured on MI355X in
   // the served mix: 1D requests of random points p50 0.49 -> 0.44 ms; the 2D
   // and 3D requests there are grids, whose order tiles or rows give already,
-  // and the sort's passes made them 1-3 % slower.
+  // and the sort's passes made them 1-3 % slower.  Where LDS beside large
+  // tables holds fewer points than kGrabMax items have, there is no order:
+  // runs of as many points as did fit, in order, measured slower than longer
+  // ones without (4 800 cells, items of 1 024 points: 841 -> 943 us; 4 200
+  // cells, 8 192 points: 1 396 -> 1 481).
   int sort_off = 0, sort_cap = 0;
   if (DIM == 1 && maxLen <= kBucketTileMax) {
     sort_cap = maxLen * kGrabMax < kBucketTileMax ? (int)maxLen * kGrabMax : kBucketTileMax;
