@@ -920,10 +920,17 @@ __global__ void __launch_bounds__(256, 2)
 
 // calc_T_simple: nStepsODE * nTimeSteps RK2 substeps (calc_2Dto2D.cu:412-445),
 // with a lookup only where some point of the wave has left the bounds of its
-// cell.  Bound by FP64 instructions: 35 a substep and point where a lookup in
-// each took 75 and a table read.  1 000 points 232 -> 150 us; 250 000: 2D type
-// I 640 -> 335, type II 470 -> 263, 3 x 5 cells 1 283 -> 395, 3D (100 000)
-// 850 -> 375; 512 x 512 grid 535 -> 480, all of it the corner's wave.
+// cell.  Bound by FP64 instructions: 35 a substep and point and 12 for the
+// bounds' test, against 75 and a table read with a lookup in each substep; but
+// to look up and form the bounds is 80.  Waves that gain nothing by bounds have
+// some point outside them nearly always (points on walls and corners, 64
+// random points in a coarse integration): after three stretches in a row that
+// ended at once (one or two in a coarse integration, where short ones are the
+// rule) come 3, 7, .. 63 substeps with a lookup each before the next one.
+// MI355X, 1 000 substeps, lookups in each / bounds always / this: 2D type I,
+// 100 000 random points 303 / 200 / 207 us, 256 x 256 grid 263 / 347 / 197,
+// 3 x 5 cells 738 / 207 / 209; 3D, 65 536 point grid 414 / 734 / 333; 1D,
+// 1 000 points 226 / 80 / 82.  100 substeps: 2D, 100 000 points 33 / 45 / 35.
 template <int DIM, int TESS, bool POW2, bool LDS>
 __global__ void __launch_bounds__(1024)
     k_simple(const double* __restrict__ pos0, double* __restrict__ out, const double* __restrict__ As,
@@ -939,24 +946,42 @@ __global__ void __launch_bounds__(1024)
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nPts) return;
   const double hh = h * 0.5;  // (as in `advance`)
-  double p[DIM], y[DIM], m[DIM], A[NE];
+  double p[DIM], A[NE];
   load_pt<DIM>(pos0, i, p);
-  CellBounds<DIM, TESS> bounds;
-  const uint64_t all = __builtin_amdgcn_read_exec();
-  uint64_t in = 0;  // lanes whose point is in the cell of their row
-  for (int s = 0; s < nSteps; s++) {
-    if (in != all) {
-      const int c = cell_of<DIM, TESS, POW2>(p, g);
+  auto lookup = [&]() {
+    const int c = cell_of<DIM, TESS, POW2>(p, g);
 #pragma unroll
-      for (int e = 0; e < NE; e++) A[e] = Atab[c * NE + e];
-      bounds.enter(c, g);
-    }
+    for (int e = 0; e < NE; e++) A[e] = Atab[c * NE + e];
+    return c;
+  };
+  auto substep = [&]() {
+    double y[DIM], m[DIM];
     affine<DIM>(y, A, p);
 #pragma unroll
     for (int d = 0; d < DIM; d++) m[d] = p[d] + hh * y[d];
     affine<DIM>(y, A, m);
 #pragma unroll
     for (int d = 0; d < DIM; d++) p[d] += y[d] * h;
+  };
+  const uint64_t all = __builtin_amdgcn_read_exec();
+  const bool coarse = nSteps <= 128;  // (few substeps in all are large ones)
+  const int kShort = TESS == TESS_I && coarse ? 2 : 1;
+  CellBounds<DIM, TESS> bounds;
+  uint64_t in = 0;  // lanes whose point is in the cell of their row
+  // substeps left, those left at the last lookup, short stretches in a row (wave-uniform)
+  int s = nSteps, last = nSteps, shorts = coarse ? 1 : -1;
+  for (; s > 0; s--) {
+    if (in != all) {
+      shorts = last - s > kShort ? 0 : shorts + 1;
+      if (shorts >= 3)
+        for (int u = (1 << (shorts < 7 ? shorts - 1 : 6)) - 1; u > 0 && s > 1; u--, s--) {
+          lookup();
+          substep();
+        }
+      last = s;
+      bounds.enter(lookup(), g);
+    }
+    substep();
     in = bounds.inside(p, g);
   }
   store_pt<DIM>(out, i, p);
