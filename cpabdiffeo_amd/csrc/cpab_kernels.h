@@ -419,10 +419,70 @@ struct CellBounds<3, TESS_I> {
   }
 };
 
+// ----------------------------------------------------------------- trip
+// One unit of the reference's step schedule for one point of a lane (all lanes of a wave in lockstep, whatever unit each is at):
+//   k == 0: y = Trel_c [p;1]; if cell(y) == c accept, else start the RK2 redo
+//           (k = nStepsODE; p and c unchanged)   (calc_2Dto2D.cu:389-401)
+//   k >  0: one RK2 midpoint substep of A_c from p (solveODE, :179-194);
+//           p = y, c = cell(y), k--.
+// Both kinds of trip share the table read, the first affine product and the
+// cell lookup, so lanes in different modes diverge only over the midpoint
+// arithmetic.  (Measured on gfx950: evaluating the midpoint in every lane
+// and selecting, or chaining several Trel proposals speculatively so their
+// lookups overlap, are both slower than this.)
+// Returns true when the step is complete (the caller advances t).
+template <int DIM, int TESS, bool POW2, bool FAST = false, bool EARLY = true>
+__device__ __forceinline__ bool trip(double* p, int& c, int& k, const double*& row, int& nfb, const double* Ttab,
+                                     const double* Atab, double h, int nS, const Geom& g) {
+  constexpr int NE = DIM * (DIM + 1);
+  const bool fast = (k == 0);
+  double y[DIM];
+  affine<DIM>(y, row, p);
+  if (!fast) {  // RK2 midpoint substep (solveODE, calc_2Dto2D.cu:182-194)
+    // The reference's h * v / 2 is fl(h v) halved; (h / 2) * v rounds the
+    // same real number h v / 2, and halving commutes with rounding, so the
+    // two agree bit for bit unless |h v / 2| is subnormal (below 2^-1022).
+    // A nonzero v = A [p; 1] is at least ~2^-53 of its largest term, so that
+    // takes table entries near 1e-290.  One multiply per coordinate fewer.
+    const double hh = h * 0.5;
+    double m[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; d++) m[d] = p[d] + hh * y[d];
+    affine<DIM>(y, row, m);
+#pragma unroll
+    for (int d = 0; d < DIM; d++) y[d] = p[d] + y[d] * h;
+  }
+  const int cy = cell_of<DIM, TESS, POW2, FAST, EARLY>(y, g);
+  // (Measured on gfx950: the state update below written as selects instead
+  // of branches ran 3-4 % slower here and 11 % slower for 256 registration
+  // chains.)
+  if (!fast) {
+#pragma unroll
+    for (int d = 0; d < DIM; d++) p[d] = y[d];
+    const bool done = --k == 0;
+    row = (done ? Ttab : Atab) + mul24(cy, NE);  // (the same row when the cell did not change)
+    c = cy;
+    return done;
+  }
+  if (cy == c) {
+#pragma unroll
+    for (int d = 0; d < DIM; d++) p[d] = y[d];
+    return true;
+  }
+  nfb++;
+  if (nS > 0) {
+    k = nS;
+    row = Atab + mul24(c, NE);
+    return false;
+  }
+  return true;  // zero substeps: the step leaves p where it was
+}
+
 // -------------------------------------------------------------- advance
-// Integrates the calling lanes (t < tb on each) to step tb by the reference's
-// schedule (calc_2Dto2D.cu:385-402: every step the Trel proposal, and when it
-// leaves the cell nS RK2 substeps instead), in two phases taken in turn:
+// Integrates the wave's lanes (t < tb on those that have a point) to step tb
+// by the reference's schedule (calc_2Dto2D.cu:385-402: every step the Trel
+// proposal, and when it leaves the cell nS RK2 substeps instead), in two phases
+// taken in turn:
 //
 //   stretch  every lane whose point is in its cell by the bounds takes Trel
 //            steps, its row and bounds in registers, until its point leaves
@@ -432,6 +492,9 @@ struct CellBounds<3, TESS_I> {
 //            and run the step's nS RK2 substeps, all of them together; some
 //            were only beside a facet and accept it.
 //
+// or in lockstep (`trip`: one proposal or substep of every lane, its cell
+// looked up and its row read each time) where phases gain nothing.
+//
 // Per point the sequence of IEEE operations is the reference's.
 //
 // What bounds calc_T is instruction issue: a wave alone on its SIMD issues an
@@ -439,24 +502,44 @@ struct CellBounds<3, TESS_I> {
 // a launch of few waves ends with its slowest one.  A step of a stretch is 24
 // VALU and 9 scalar instructions (2D type I: 8 the affine product, 8 the
 // bounds, 8 the update) against 36 and 20 and LDS latency for a trip in
-// lockstep (one unit, proposal or substep, of every lane, its cell looked up
-// and its row read each time; see `trip`), or 52 when some lane of the wave
-// is at a redone step.  The loop has no divergent branch: lanes that have
-// left stay where they are by selects.  A redo costs about as much as 20
-// steps of a stretch however many lanes share it, and a lane that waits for
-// company delays the wave's end: hence kSeg (16, 24, 32 and 100 steps: 2D
-// 2 000 000 points 534, 470, 448 us; 3D volume warp 351, 319, 308, 341 us).
-// On MI355X, lockstep -> this: 2D random points, 1 000: 51 -> 41 us, 65 536:
-// 56 -> 45, 2 000 000: 606 -> 430; grids, 512 x 512: 67 -> 67 (its slowest
-// waves cross many facets), 2048 x 2048: 735 -> 580; 640 x 480 with fields
-// that leave the image 175 -> 137; 1D, 10^6 points of 50 cells 274 -> 195;
-// 3D, 64 x 80 x 96 volume 331 -> 308.
+// lockstep, or 52 when some lane of the wave is at a redone step.  The loop has
+// no divergent branch: lanes that have left stay where they are by selects.  A
+// redo costs about as much as 20 steps of a stretch however many lanes share
+// it, and a lane that waits for company delays the wave's end: hence kSeg (16,
+// 24, 32 and 100 steps: 2D 2 000 000 points 534, 470, 448 us; 3D volume warp
+// 351, 319, 308, 341 us).  On MI355X, lockstep -> phases: 2D random points,
+// 1 000: 51 -> 41 us, 65 536: 56 -> 45, 2 000 000: 606 -> 430; grids, 512 x
+// 512: 67 -> 67 (its slowest waves cross many facets), 2048 x 2048: 735 -> 580;
+// 640 x 480 with fields that leave the image 175 -> 137; 1D, 10^6 points of 50
+// cells 274 -> 195; 3D, 64 x 80 x 96 volume 331 -> 308.
+//
+// Lockstep (lock: its trips still to run; a lane may return in the middle of a
+// step, k substeps to go) instead of phases:
+//   * all the way where the whole integration is at most kFewSubsteps substeps:
+//     its steps are so large that points leave their cells every few of them,
+//     and a redo is too short for waiting to pay.  100 000 points, phases ->
+//     lockstep: 30 steps of 3, 2D 42 -> 29 us, 3D 60 -> 39; 100 of 1, 16 x 16
+//     cells and a fast field 206 -> 95.  Beyond it phases: 100 of 4 and 30 of
+//     10 are 13 % faster in phases (median of 54 calls).
+//   * a window of kLock trips, doubled while they follow each other, where no
+//     lane's point is inside its bounds (on walls, at rest).  Rounds of one step
+//     each, all lanes waiting for the redo of whichever left its cell, took
+//     longer where different lanes leave at different steps: 2D grids in 100
+//     steps of 10 up to 1.2 times, 3D grids of 262 144 points in 20 steps of 100
+//     940 us against 500 (4 x 4 x 4 boxes), in 30 of 10 1.2 times.  But a trip
+//     of a 3D lane that redoes most of its steps (points drawn to an edge of
+//     the tessellation) costs more than a round: 56 x 30 x 50 volume, 100 steps
+//     of 10, 720 us in rounds, 930 in windows.  Hence rounds in 3D from 64 steps
+//     of five substeps on.
 //
 // more: the caller has further points for lanes that finish; then it returns
 // as soon as `refill` lanes have.
 constexpr int kSeg = 32;
 constexpr int kSegTraj = 12;  // calc_trajectory: lanes far apart in steps store to as many rows (16: +3 %, 8: +6 %)
 constexpr int kRefill = 8;
+constexpr int kLock = 16;          // trips in lockstep before phases are tried again
+constexpr int kTrips = 2;          // trips between two looks at the lanes that are done (1: 8 % slower; 4: the same)
+constexpr int kFewSubsteps = 100;  // of an integration in lockstep from the start
 
 // The point at the domain's corner (0, 0).  With zero velocity on the walls
 // its velocity is zero up to rounding: it drifts ~1e-16 out of the domain and
@@ -552,9 +635,9 @@ __device__ __forceinline__ void corner_steps(double* p, int& c, int& t, int tb, 
 }
 
 template <int DIM, int TESS, bool POW2, int MODE>
-__device__ __forceinline__ void advance(double* p, int& c, int& t, int tb, int& nfb, const double* Ttab,
-                                        const double* Atab, double h, int nS, const Geom& g, bool more_,
-                                        int refill, double* __restrict__ traj, int64_t nPts) {
+__device__ __forceinline__ void advance(double* p, int& c, int& k, int& t, int tb, int& nfb, int& lock,
+                                        const double* Ttab, const double* Atab, double h, int nS, const Geom& g,
+                                        bool more, int refill, double* __restrict__ traj, int64_t nPts) {
   constexpr int NE = DIM * (DIM + 1);
   // The reference's h * v / 2 is fl(h v) halved; (h / 2) * v rounds the same
   // real number h v / 2, and halving commutes with rounding, so the two agree
@@ -562,17 +645,15 @@ __device__ __forceinline__ void advance(double* p, int& c, int& t, int tb, int& 
   // v = A [p; 1] is at least ~2^-53 of its largest term, so that takes table
   // entries near 1e-290.  One multiply per coordinate fewer.
   const double hh = h * 0.5;
-  const int nAll = __popcll(__builtin_amdgcn_read_exec());
   constexpr int seg = MODE == 1 ? kSegTraj : kSeg;
-  const bool more = __builtin_amdgcn_readfirstlane((int)more_) != 0;  // (wave-uniform: kept in scalar registers)
-  int cool = 0;  // rounds without a stretch (wave-uniform)
+  const bool windows = DIM < 3 || tb < 64 || nS < 5;
+  int cool = 0, window = kLock;  // rounds without a stretch, trips of the next window (wave-uniform)
   for (;;) {
     const uint64_t todo = ballot(t < tb);
     const int nTodo = __popcll(todo);
-    if (nTodo == 0 || (more && nAll - nTodo >= refill)) break;
-    bool waits = t < tb;  // the lane takes part in the redo phase
-    if (DIM == 2 && TESS == TESS_I && POW2 && nTodo == 1 && cool > 0) {  // one lane left, and no stretch for it
-      if (waits && (c == 0 || c == 3) && __builtin_fabs(p[0]) < 0.125 * g.inc_x &&
+    if (nTodo == 0 || (more && 64 - nTodo >= refill)) break;
+    if (DIM == 2 && TESS == TESS_I && POW2 && nTodo == 1 && lock > 0) {  // one lane left, and no stretch for it
+      if (t < tb && k == 0 && (c == 0 || c == 3) && __builtin_fabs(p[0]) < 0.125 * g.inc_x &&
           __builtin_fabs(p[1]) < 0.125 * g.inc_y) {
         corner_steps(
             p, c, t, tb, Ttab, Atab, h, nS, g, [](int, int) {}, [](int) {},
@@ -580,10 +661,30 @@ __device__ __forceinline__ void advance(double* p, int& c, int& t, int tb, int& 
               nfb += redo ? 1 : 0;
               if (MODE == 1) store_pt<2>(traj, (int64_t)step * nPts, q);
             });
-        waits = false;
       }
     }
-    if (cool > 0) {
+    if (lock > 0) {
+      const double* row = (k == 0 ? Ttab : Atab) + mul24(c, NE);
+      for (;;) {
+        bool on = t < tb && (lock > 0 || k > 0);
+        if (ballot(on) == 0) break;
+        for (int u = 0; u < kTrips; u++) {
+          if (on) {
+            if (trip<DIM, TESS, POW2, true>(p, c, k, row, nfb, Ttab, Atab, h, nS, g)) {
+              if (MODE == 1) store_pt<DIM>(traj, (int64_t)t * nPts, p);
+              t++;
+            }
+            on = t < tb && (lock > 0 || k > 0);
+          }
+        }
+        lock -= kTrips;
+        if (more && 64 - __popcll(ballot(t < tb)) >= refill) break;
+      }
+      if (more && lock <= 0) lock = ballot(k > 0) != 0 ? 1 : 0;
+      continue;
+    }
+    bool waits = t < tb;  // the lane takes part in the redo phase
+    if (DIM == 3 && cool > 0) {
       cool--;
     } else {
       CellBounds<DIM, TESS> B;
@@ -593,7 +694,15 @@ __device__ __forceinline__ void advance(double* p, int& c, int& t, int tb, int& 
       for (int e = 0; e < NE; e++) R[e] = row[e];
       B.enter(c, g);
       uint64_t go = B.inside(p, g) & todo;  // the lanes of the stretch
-      if (go == 0) cool = 8;
+      if (go == 0) {
+        if (windows) {
+          lock = window;
+          window = window < 256 ? 2 * window : 256;
+          continue;
+        }
+        cool = 8;
+      }
+      window = kLock;
       for (;;) {
         const int lim = tb - t < seg ? tb : t + seg;
         while (go != 0) {
@@ -608,7 +717,7 @@ __device__ __forceinline__ void advance(double* p, int& c, int& t, int tb, int& 
         }
         waits = t < lim;
         go = ballot(t < tb);  // with no lane waiting the cells are still the same
-        if (go == 0 || ballot(waits) != 0 || (more && nAll - __popcll(go) >= refill)) break;
+        if (go == 0 || ballot(waits) != 0 || (more && 64 - __popcll(go) >= refill)) break;
       }
     }
     if (waits) {
@@ -729,10 +838,13 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* curso
   // instances, 8 instead of 16: 14.3 -> 13.9 ms, 32: 16.7; 64: 15.3)
   const int refill = gord.w > 0 ? 64 : kRefill;
   double p[DIM];
-  int c = 0, t = 0, nfb = 0;
+#pragma unroll
+  for (int d = 0; d < DIM; d++) p[d] = 0.0;
+  int c = 0, k = 0, t = nT, nfb = 0;  // (an idle lane is at step nT)
   int64_t my = 0;
   bool active = false, more = true;
   int taken = 0;  // points the cursor leaves out
+  int lock = (int64_t)nT * nS <= kFewSubsteps ? 1 << 30 : 0;  // trips in lockstep still to run (wave-uniform)
   if (DIM == 2 && TESS == TESS_I && POW2 && MODE == 0 && corner != 0) {
     bool near = false;
     if (gord.w > 0) {
@@ -744,6 +856,7 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* curso
       if (!near) return;
       active = threadIdx.x == 0;
       more = false;
+      t = active ? 0 : nT;
       c = cell_of<DIM, TESS, POW2>(p, g);
     }
     taken = near ? 1 : 0;
@@ -773,8 +886,7 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* curso
       more = next + taken + __popcll(idle) < n;
     }
     if (ballot(active) == 0) break;
-    if (!active || t >= nT) continue;
-    advance<DIM, TESS, POW2, MODE>(p, c, t, nT, nfb, Ttab, Atab, h, nS, g, more, refill,
+    advance<DIM, TESS, POW2, MODE>(p, c, k, t, nT, nfb, lock, Ttab, Atab, h, nS, g, more, refill,
                                    MODE == 1 ? out + my * DIM : nullptr, nPts);
   }
 }

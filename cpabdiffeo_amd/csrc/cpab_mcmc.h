@@ -47,69 +47,12 @@
 
 namespace cpab {
 
-// ----------------------------------------------------------------- trip
-// The registration step integrates in lockstep (calc_T's two phases, `advance`,
-// measured 6 % slower here: 79 instead of 63 VGPRs leave fewer waves, and a
-// wave that ends later tells later slots later that they are not needed).
-// One unit of the reference's step schedule for one point of a lane (all lanes of a wave in lockstep, whatever unit each is at):
-//   k == 0: y = Trel_c [p;1]; if cell(y) == c accept, else start the RK2 redo
-//           (k = nStepsODE; p and c unchanged)   (calc_2Dto2D.cu:389-401)
-//   k >  0: one RK2 midpoint substep of A_c from p (solveODE, :179-194);
-//           p = y, c = cell(y), k--.
-// Both kinds of trip share the table read, the first affine product and the
-// cell lookup, so lanes in different modes diverge only over the midpoint
-// arithmetic.  (Measured on gfx950: evaluating the midpoint in every lane
-// and selecting, or chaining several Trel proposals speculatively so their
-// lookups overlap, are both slower than this.)
-// Returns true when the step is complete (the caller advances t).
-template <int DIM, int TESS, bool POW2, bool FAST = false, bool EARLY = true>
-__device__ __forceinline__ bool trip(double* p, int& c, int& k, const double*& row, int& nfb, const double* Ttab,
-                                     const double* Atab, double h, int nS, const Geom& g) {
-  constexpr int NE = DIM * (DIM + 1);
-  const bool fast = (k == 0);
-  double y[DIM];
-  affine<DIM>(y, row, p);
-  if (!fast) {  // RK2 midpoint substep (solveODE, calc_2Dto2D.cu:182-194)
-    // The reference's h * v / 2 is fl(h v) halved; (h / 2) * v rounds the
-    // same real number h v / 2, and halving commutes with rounding, so the
-    // two agree bit for bit unless |h v / 2| is subnormal (below 2^-1022).
-    // A nonzero v = A [p; 1] is at least ~2^-53 of its largest term, so that
-    // takes table entries near 1e-290.  One multiply per coordinate fewer.
-    const double hh = h * 0.5;
-    double m[DIM];
-#pragma unroll
-    for (int d = 0; d < DIM; d++) m[d] = p[d] + hh * y[d];
-    affine<DIM>(y, row, m);
-#pragma unroll
-    for (int d = 0; d < DIM; d++) y[d] = p[d] + y[d] * h;
-  }
-  const int cy = cell_of<DIM, TESS, POW2, FAST, EARLY>(y, g);
-  // (Measured on gfx950: the state update below written as selects instead
-  // of branches ran 3-4 % slower here and 11 % slower for 256 registration
-  // chains.)
-  if (!fast) {
-#pragma unroll
-    for (int d = 0; d < DIM; d++) p[d] = y[d];
-    const bool done = --k == 0;
-    row = (done ? Ttab : Atab) + mul24(cy, NE);  // (the same row when the cell did not change)
-    c = cy;
-    return done;
-  }
-  if (cy == c) {
-#pragma unroll
-    for (int d = 0; d < DIM; d++) p[d] = y[d];
-    return true;
-  }
-  nfb++;
-  if (nS > 0) {
-    k = nS;
-    row = Atab + mul24(c, NE);
-    return false;
-  }
-  return true;  // zero substeps: the step leaves p where it was
-}
-
 // ------------------------------------------------------------ lone lane
+// The registration step integrates in lockstep (`trip`); calc_T's two phases
+// (`advance`) measured 6 % slower here: 79 instead of 63 VGPRs leave fewer
+// waves, and a wave that ends later tells later slots later that they are not
+// needed.
+//
 // A wave left with a single unfinished lane runs one dependent chain of
 // instructions, so its trips cost their latency (a dependent FP64 operation
 // takes 16-22 cycles on MI355X), not their issue.  The point that gets there
