@@ -536,6 +536,15 @@ __device__ __forceinline__ bool trip(double* p, int& c, int& k, const double*& r
 // as soon as `refill` lanes have.
 constexpr int kSeg = 32;
 constexpr int kSegTraj = 12;  // calc_trajectory: lanes far apart in steps store to as many rows (16: +3 %, 8: +6 %)
+// calc_trajectory, more rows than the 256 MiB cache holds: the steps that a lane
+// may be ahead of its wave's last.  Rows are written a point at a time, so a
+// line stays in a cache until the wave's lanes have all been there, and a lane
+// falls behind by a segment whenever it changes cell.  100 000 points, 1 000
+// steps of 1 substep (1.6 GB), no bound / 64 / 32 / 16 steps: 1D, 50 cells 958,
+// 726, 375, 243 us (in lockstep 439); 2D, 500 steps of 3 431, 441, 391, 230
+// (349).  500 000 2D points, 100 steps of 10: 494 -> 376 us.
+constexpr int kSpread = 16;
+constexpr int64_t kCacheBytes = 256 << 20;
 constexpr int kRefill = 8;
 constexpr int kLock = 16;          // trips in lockstep before phases are tried again
 constexpr int kTrips = 2;          // trips between two looks at the lanes that are done (1: 8 % slower; 4: the same)
@@ -637,7 +646,8 @@ __device__ __forceinline__ void corner_steps(double* p, int& c, int& t, int tb, 
 template <int DIM, int TESS, bool POW2, int MODE>
 __device__ __forceinline__ void advance(double* p, int& c, int& k, int& t, int tb, int& nfb, int& lock,
                                         const double* Ttab, const double* Atab, double h, int nS, const Geom& g,
-                                        bool more, int refill, double* __restrict__ traj, int64_t nPts) {
+                                        bool more, int refill, double* __restrict__ traj, int64_t nPts,
+                                        bool far) {
   constexpr int NE = DIM * (DIM + 1);
   // The reference's h * v / 2 is fl(h v) halved; (h / 2) * v rounds the same
   // real number h v / 2, and halving commutes with rounding, so the two agree
@@ -704,7 +714,16 @@ __device__ __forceinline__ void advance(double* p, int& c, int& k, int& t, int t
       }
       window = kLock;
       for (;;) {
-        const int lim = tb - t < seg ? tb : t + seg;
+        int lim = tb - t < seg ? tb : t + seg;
+        if (MODE == 1 && far) {  // (uniform)
+          int m = t;
+#pragma unroll
+          for (int o = 32; o > 0; o >>= 1) {
+            const int x = __shfl_xor(m, o, 64);
+            m = x < m ? x : m;
+          }
+          lim = lim < m + kSpread ? lim : m + kSpread;
+        }
         while (go != 0) {
           double y[DIM];
           affine<DIM>(y, R, p);
@@ -887,7 +906,8 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* curso
     }
     if (ballot(active) == 0) break;
     advance<DIM, TESS, POW2, MODE>(p, c, k, t, nT, nfb, lock, Ttab, Atab, h, nS, g, more, refill,
-                                   MODE == 1 ? out + my * DIM : nullptr, nPts);
+                                   MODE == 1 ? out + my * DIM : nullptr, nPts,
+                                   MODE == 1 && nT * nPts > kCacheBytes / (8 * DIM));
   }
 }
 
