@@ -479,8 +479,8 @@ __device__ __forceinline__ bool trip(double* p, int& c, int& k, const double*& r
 }
 
 // -------------------------------------------------------------- advance
-// Integrates the wave's lanes (t < tb on those that have a point) to step tb
-// by the reference's schedule (calc_2Dto2D.cu:385-402: every step the Trel
+// Integrates the calling lanes (t < tb on each that has a point) to step tb by
+// the reference's schedule (calc_2Dto2D.cu:385-402: every step the Trel
 // proposal, and when it leaves the cell nS RK2 substeps instead), in two phases
 // taken in turn:
 //
@@ -492,8 +492,9 @@ __device__ __forceinline__ bool trip(double* p, int& c, int& k, const double*& r
 //            and run the step's nS RK2 substeps, all of them together; some
 //            were only beside a facet and accept it.
 //
-// or in lockstep (`trip`: one proposal or substep of every lane, its cell
-// looked up and its row read each time) where phases gain nothing.
+// or, for coarse integrations (lockstep_pays), in lockstep (advance_lockstep):
+// one proposal or substep of every lane at a time, its cell looked up and its
+// row read each time (`trip`).
 //
 // Per point the sequence of IEEE operations is the reference's.
 //
@@ -513,25 +514,6 @@ __device__ __forceinline__ bool trip(double* p, int& c, int& k, const double*& r
 // 640 x 480 with fields that leave the image 175 -> 137; 1D, 10^6 points of 50
 // cells 274 -> 195; 3D, 64 x 80 x 96 volume 331 -> 308.
 //
-// Lockstep (lock: its trips still to run; a lane may return in the middle of a
-// step, k substeps to go) instead of phases:
-//   * all the way where the whole integration is at most kFewSubsteps substeps:
-//     its steps are so large that points leave their cells every few of them,
-//     and a redo is too short for waiting to pay.  100 000 points, phases ->
-//     lockstep: 30 steps of 3, 2D 42 -> 29 us, 3D 60 -> 39; 100 of 1, 16 x 16
-//     cells and a fast field 206 -> 95.  Beyond it phases: 100 of 4 and 30 of
-//     10 are 13 % faster in phases (median of 54 calls).
-//   * a window of kLock trips, doubled while they follow each other, where no
-//     lane's point is inside its bounds (on walls, at rest).  Rounds of one step
-//     each, all lanes waiting for the redo of whichever left its cell, took
-//     longer where different lanes leave at different steps: 2D grids in 100
-//     steps of 10 up to 1.2 times, 3D grids of 262 144 points in 20 steps of 100
-//     940 us against 500 (4 x 4 x 4 boxes), in 30 of 10 1.2 times.  But a trip
-//     of a 3D lane that redoes most of its steps (points drawn to an edge of
-//     the tessellation) costs more than a round: 56 x 30 x 50 volume, 100 steps
-//     of 10, 720 us in rounds, 930 in windows.  Hence rounds in 3D from 64 steps
-//     of five substeps on.
-//
 // more: the caller has further points for lanes that finish; then it returns
 // as soon as `refill` lanes have.
 constexpr int kSeg = 32;
@@ -546,9 +528,21 @@ constexpr int kSegTraj = 12;  // calc_trajectory: lanes far apart in steps store
 constexpr int kSpread = 16;
 constexpr int64_t kCacheBytes = 256 << 20;
 constexpr int kRefill = 8;
-constexpr int kLock = 16;          // trips in lockstep before phases are tried again
-constexpr int kTrips = 2;          // trips between two looks at the lanes that are done (1: 8 % slower; 4: the same)
-constexpr int kFewSubsteps = 100;  // of an integration in lockstep from the start
+constexpr int kTrips = 2;  // trips in lockstep between two looks at the lanes that are done (1: 8 % slower; 4: the same)
+
+// Lockstep instead of phases for integrations of few large steps: points leave
+// their cells every few of them, so a stretch is short, and every lane waits for
+// the redo of whichever left.  Up to 100 substeps in all, phases -> lockstep,
+// 100 000 points: 30 steps of 3, 2D 42 -> 29 us, 3D 60 -> 39; 100 steps of 1,
+// 16 x 16 cells and a fast field 206 -> 95.  In 3D below 64 steps whatever the
+// substeps, as more of a wave's points leave at each step there: grids of
+// 262 144 points, 4 x 4 x 4 boxes, 20 steps of 100 938 -> 500 us, 30 of 10 134 ->
+// 91 (random points within 16 % either way).  Beyond both, phases: 1D and 2D in
+// 30 steps of 10 take 0.60 of the time of an older lockstep kernel (median of
+// 36 calls), lockstep 0.73; 100 steps of 4 0.63 and 0.75.
+__host__ __device__ constexpr bool lockstep_pays(int dim, int nT, int nS) {
+  return (int64_t)nT * nS <= 100 || (dim == 3 && nT < 64);
+}
 
 // The point at the domain's corner (0, 0).  With zero velocity on the walls
 // its velocity is zero up to rounding: it drifts ~1e-16 out of the domain and
@@ -644,10 +638,9 @@ __device__ __forceinline__ void corner_steps(double* p, int& c, int& t, int tb, 
 }
 
 template <int DIM, int TESS, bool POW2, int MODE>
-__device__ __forceinline__ void advance(double* p, int& c, int& k, int& t, int tb, int& nfb, int& lock,
-                                        const double* Ttab, const double* Atab, double h, int nS, const Geom& g,
-                                        bool more, int refill, double* __restrict__ traj, int64_t nPts,
-                                        bool far) {
+__device__ __forceinline__ void advance(double* p, int& c, int& t, int tb, int& nfb, const double* Ttab,
+                                        const double* Atab, double h, int nS, const Geom& g, bool more_,
+                                        int refill, double* __restrict__ traj, int64_t nPts, bool far) {
   constexpr int NE = DIM * (DIM + 1);
   // The reference's h * v / 2 is fl(h v) halved; (h / 2) * v rounds the same
   // real number h v / 2, and halving commutes with rounding, so the two agree
@@ -655,15 +648,17 @@ __device__ __forceinline__ void advance(double* p, int& c, int& k, int& t, int t
   // v = A [p; 1] is at least ~2^-53 of its largest term, so that takes table
   // entries near 1e-290.  One multiply per coordinate fewer.
   const double hh = h * 0.5;
+  const int nAll = __popcll(__builtin_amdgcn_read_exec());
   constexpr int seg = MODE == 1 ? kSegTraj : kSeg;
-  const bool windows = DIM < 3 || tb < 64 || nS < 5;
-  int cool = 0, window = kLock;  // rounds without a stretch, trips of the next window (wave-uniform)
+  const bool more = __builtin_amdgcn_readfirstlane((int)more_) != 0;  // (wave-uniform: kept in scalar registers)
+  int cool = 0;  // rounds without a stretch (wave-uniform)
   for (;;) {
     const uint64_t todo = ballot(t < tb);
     const int nTodo = __popcll(todo);
-    if (nTodo == 0 || (more && 64 - nTodo >= refill)) break;
-    if (DIM == 2 && TESS == TESS_I && POW2 && nTodo == 1 && lock > 0) {  // one lane left, and no stretch for it
-      if (t < tb && k == 0 && (c == 0 || c == 3) && __builtin_fabs(p[0]) < 0.125 * g.inc_x &&
+    if (nTodo == 0 || (more && nAll - nTodo >= refill)) break;
+    bool waits = t < tb;  // the lane takes part in the redo phase
+    if (DIM == 2 && TESS == TESS_I && POW2 && nTodo == 1 && cool > 0) {  // one lane left, and no stretch for it
+      if (waits && (c == 0 || c == 3) && __builtin_fabs(p[0]) < 0.125 * g.inc_x &&
           __builtin_fabs(p[1]) < 0.125 * g.inc_y) {
         corner_steps(
             p, c, t, tb, Ttab, Atab, h, nS, g, [](int, int) {}, [](int) {},
@@ -671,30 +666,10 @@ __device__ __forceinline__ void advance(double* p, int& c, int& k, int& t, int t
               nfb += redo ? 1 : 0;
               if (MODE == 1) store_pt<2>(traj, (int64_t)step * nPts, q);
             });
+        waits = false;
       }
     }
-    if (lock > 0) {
-      const double* row = (k == 0 ? Ttab : Atab) + mul24(c, NE);
-      for (;;) {
-        bool on = t < tb && (lock > 0 || k > 0);
-        if (ballot(on) == 0) break;
-        for (int u = 0; u < kTrips; u++) {
-          if (on) {
-            if (trip<DIM, TESS, POW2, true>(p, c, k, row, nfb, Ttab, Atab, h, nS, g)) {
-              if (MODE == 1) store_pt<DIM>(traj, (int64_t)t * nPts, p);
-              t++;
-            }
-            on = t < tb && (lock > 0 || k > 0);
-          }
-        }
-        lock -= kTrips;
-        if (more && 64 - __popcll(ballot(t < tb)) >= refill) break;
-      }
-      if (more && lock <= 0) lock = ballot(k > 0) != 0 ? 1 : 0;
-      continue;
-    }
-    bool waits = t < tb;  // the lane takes part in the redo phase
-    if (DIM == 3 && cool > 0) {
+    if (cool > 0) {
       cool--;
     } else {
       CellBounds<DIM, TESS> B;
@@ -704,18 +679,10 @@ __device__ __forceinline__ void advance(double* p, int& c, int& k, int& t, int t
       for (int e = 0; e < NE; e++) R[e] = row[e];
       B.enter(c, g);
       uint64_t go = B.inside(p, g) & todo;  // the lanes of the stretch
-      if (go == 0) {
-        if (windows) {
-          lock = window;
-          window = window < 256 ? 2 * window : 256;
-          continue;
-        }
-        cool = 8;
-      }
-      window = kLock;
+      if (go == 0) cool = 8;
       for (;;) {
         int lim = tb - t < seg ? tb : t + seg;
-        if (MODE == 1 && far) {  // (uniform)
+        if (MODE == 1 && far) {  // (uniform; every lane of the wave is here, those without a point at t >= tb)
           int m = t;
 #pragma unroll
           for (int o = 32; o > 0; o >>= 1) {
@@ -736,7 +703,7 @@ __device__ __forceinline__ void advance(double* p, int& c, int& k, int& t, int t
         }
         waits = t < lim;
         go = ballot(t < tb);  // with no lane waiting the cells are still the same
-        if (go == 0 || ballot(waits) != 0 || (more && 64 - __popcll(go) >= refill)) break;
+        if (go == 0 || ballot(waits) != 0 || (more && nAll - __popcll(go) >= refill)) break;
       }
     }
     if (waits) {
@@ -763,6 +730,30 @@ __device__ __forceinline__ void advance(double* p, int& c, int& k, int& t, int t
       }
       if (MODE == 1) store_pt<DIM>(traj, (int64_t)t * nPts, p);
       t++;
+    }
+  }
+}
+
+// The same in lockstep.  k: substeps that a lane has to go in its step (0
+// between steps), kept from call to call.  Every lane of the wave calls it, those
+// without a point with t >= tb.
+template <int DIM, int TESS, bool POW2, int MODE>
+__device__ __forceinline__ void advance_lockstep(double* p, int& c, int& k, int& t, int tb, int& nfb,
+                                                 const double* Ttab, const double* Atab, double h, int nS,
+                                                 const Geom& g, bool more, int refill, double* __restrict__ traj,
+                                                 int64_t nPts) {
+  constexpr int NE = DIM * (DIM + 1);
+  const double* row = (k == 0 ? Ttab : Atab) + mul24(c, NE);
+  for (;;) {
+    const int nTodo = __popcll(ballot(t < tb));
+    if (nTodo == 0 || (more && 64 - nTodo >= refill)) break;
+    for (int u = 0; u < kTrips; u++) {
+      if (t < tb) {
+        if (trip<DIM, TESS, POW2, true>(p, c, k, row, nfb, Ttab, Atab, h, nS, g)) {
+          if (MODE == 1) store_pt<DIM>(traj, (int64_t)t * nPts, p);
+          t++;
+        }
+      }
     }
   }
 }
@@ -844,13 +835,12 @@ __device__ __forceinline__ GridOrder grid_order(int w, int64_t n) {
 // it out (1): it may be `corner_steps`'s, and among 63 neighbours it took one
 // step to their stretch of 32 until they were done (512 x 512 grid with a
 // flipping corner 195 -> 163 us; other launches, one block more, the same).
-template <int DIM, int TESS, bool POW2, int MODE>
-__device__ __forceinline__ void integrate_range(int64_t begin, int n, int* cursor, const double* __restrict__ pos0,
+template <int DIM, int TESS, bool POW2, int MODE, bool LOCK>
+__device__ __forceinline__ void integrate_points(int64_t begin, int n, int* cursor, const double* __restrict__ pos0,
                                                 double* __restrict__ out, const double* Ttab, const double* Atab,
                                                 double h, int nT, int nS, int64_t nPts, const Geom& g,
-                                                int32_t* __restrict__ nfb_out, const GridOrder& gord = GridOrder(),
-                                                int64_t gbase = 0, const uint16_t* lord = nullptr,
-                                                int corner = 0) {
+                                                int32_t* __restrict__ nfb_out, const GridOrder& gord,
+                                                int64_t gbase, const uint16_t* lord, int corner) {
   // a grid's tiles are 64 neighbouring points that need similar work, so a
   // wave takes one after another (2048 x 2048 points: 750 -> 610 us); other
   // waves take the next points as soon as kRefill lanes are free (256 batched
@@ -863,7 +853,6 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* curso
   int64_t my = 0;
   bool active = false, more = true;
   int taken = 0;  // points the cursor leaves out
-  int lock = (int64_t)nT * nS <= kFewSubsteps ? 1 << 30 : 0;  // trips in lockstep still to run (wave-uniform)
   if (DIM == 2 && TESS == TESS_I && POW2 && MODE == 0 && corner != 0) {
     bool near = false;
     if (gord.w > 0) {
@@ -905,14 +894,37 @@ __device__ __forceinline__ void integrate_range(int64_t begin, int n, int* curso
       more = next + taken + __popcll(idle) < n;
     }
     if (ballot(active) == 0) break;
-    advance<DIM, TESS, POW2, MODE>(p, c, k, t, nT, nfb, lock, Ttab, Atab, h, nS, g, more, refill,
-                                   MODE == 1 ? out + my * DIM : nullptr, nPts,
-                                   MODE == 1 && nT * nPts > kCacheBytes / (8 * DIM));
+    if (LOCK) {
+      advance_lockstep<DIM, TESS, POW2, MODE>(p, c, k, t, nT, nfb, Ttab, Atab, h, nS, g, more, refill,
+                                              MODE == 1 ? out + my * DIM : nullptr, nPts);
+    } else if (MODE == 1 || (active && t < nT)) {  // (calc_trajectory's compares the lanes' steps: all of them call it)
+      advance<DIM, TESS, POW2, MODE>(p, c, t, nT, nfb, Ttab, Atab, h, nS, g, more, refill,
+                                     MODE == 1 ? out + my * DIM : nullptr, nPts,
+                                     MODE == 1 && nT * nPts > kCacheBytes / (8 * DIM));
+    }
   }
 }
 
-// Launches of k_integrate that have a block ahead of the points' own, for the
-// corner's point (the cases of `corner_steps`).
+// (Two copies of the loop: phases and lockstep in one, chosen wave by wave as
+// points left the bounds of their cells, cost the phases 2-10 %, and up to 30 %
+// where a wave's last lane redoes its steps.)
+template <int DIM, int TESS, bool POW2, int MODE>
+__device__ __forceinline__ void integrate_range(int64_t begin, int n, int* cursor, const double* __restrict__ pos0,
+                                                double* __restrict__ out, const double* Ttab, const double* Atab,
+                                                double h, int nT, int nS, int64_t nPts, const Geom& g,
+                                                int32_t* __restrict__ nfb_out, const GridOrder& gord = GridOrder(),
+                                                int64_t gbase = 0, const uint16_t* lord = nullptr,
+                                                int corner = 0) {
+  if (lockstep_pays(DIM, nT, nS))  // (kernel arguments: uniform)
+    integrate_points<DIM, TESS, POW2, MODE, true>(begin, n, cursor, pos0, out, Ttab, Atab, h, nT, nS, nPts, g, nfb_out,
+                                                  gord, gbase, lord, corner);
+  else
+    integrate_points<DIM, TESS, POW2, MODE, false>(begin, n, cursor, pos0, out, Ttab, Atab, h, nT, nS, nPts, g, nfb_out,
+                                                   gord, gbase, lord, corner);
+}
+
+// Launches of k_integrate that have a block ahead of the points' own, for
+// the corner's point (the cases of `corner_steps`).
 constexpr bool has_corner_block(int dim, int tess, bool pow2, int mode) {
   return mode == 0 && dim == 2 && tess == TESS_I && pow2;
 }

@@ -1,11 +1,11 @@
-"""calc_T's lockstep: integrations of few substeps, and windows of trips.
+"""calc_T's two paths, in lockstep and in phases, around where one gives way to the other.
 
 A wave integrates in lockstep where the whole integration is at most 100
-substeps, and for a window of trips where no lane's point is inside the bounds
-of its cell; a lane may then wait for new points of its wave in the middle of
-a step.  Step counts around 100 substeps (and without substeps or steps),
-points on walls, at rest, calm and changing cell at most steps; single calls,
-and one wave that takes all the points of a batch's tile or of a work item.
+substeps, in 3D below 64 steps; a lane may then wait for new points of its wave
+in the middle of a step.  Step counts around both limits (and without substeps
+or steps), points on walls, at rest, calm and changing cell at most steps;
+single calls, and one wave that takes all the points of a batch's tile or of a
+work item.
 End points, fallback counts and trajectories against the oracle, bit for bit
 (cpab/gpu/calc_2Dto2D.cu:348-408)."""
 import ctypes
@@ -20,7 +20,7 @@ from test_gpu_simple_walls import CASES, points, tables
 
 pytestmark = pytest.mark.gpu
 
-STEPS = [(0, 5), (1, 5), (3, 33), (10, 10), (100, 1), (101, 1), (10, 11), (7, 0), (2, 60), (40, 4), (120, 10)]
+STEPS = [(0, 5), (1, 5), (3, 33), (10, 10), (100, 1), (101, 1), (10, 11), (7, 0), (2, 60), (40, 4), (63, 4), (64, 4), (120, 10)]
 
 
 @pytest.mark.parametrize("dim,tess,nCs,extent", CASES)
