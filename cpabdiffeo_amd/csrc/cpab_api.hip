@@ -224,14 +224,22 @@ int launch_integrate_t(cpab_ctx* ctx, int mode, const Shape& s, const double* po
   if (mode == 0) {
     auto k = k_integrate<DIM, TESS, POW2, LDS, 0>;
     allow_lds(k, s.lds);
-    const int64_t blocks = s.grid + (has_corner_block(DIM, TESS, POW2, 0) ? 1 : 0);
+    // The corner's block where the chip holds it beside the others (20 waves a
+    // CU, see k_integrate's bound): one block more than that begins a round of
+    // its own, in which large tables are staged again (16 x 16 cells, 512 x 512
+    // grid, a block a CU: one step 11.1 us, with a 257th block 15.4).
+    int64_t room = (int64_t)1280 / s.block;
+    if (s.lds > 0) room = std::min(room, (int64_t)((size_t)ctx->max_lds / (s.lds + kOwnLds)));
+    room *= ctx->n_cu;
+    const int corner = has_corner_block(DIM, TESS, POW2, 0) && nT >= kOrderSteps && s.grid % room != 0 ? 1 : 0;
+    const int64_t blocks = s.grid + corner;
     hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(s.block), s.lds, ctx->stream, pos0, out, Trels, As, h, nT, nS,
-                       nPts, g, nC, s.ptsPerWave, nfb, ps);
+                       nPts, g, nC, s.ptsPerWave, nfb, ps, corner);
   } else {
     auto k = k_integrate<DIM, TESS, POW2, LDS, 1>;
     allow_lds(k, s.lds);
     hipLaunchKernelGGL(k, dim3((unsigned)s.grid), dim3(s.block), s.lds, ctx->stream, pos0, out, Trels, As, h, nT, nS,
-                       nPts, g, nC, s.ptsPerWave, nfb, ps);
+                       nPts, g, nC, s.ptsPerWave, nfb, ps, 0);
   }
   HIP_OK(ctx, hipGetLastError());
   return CPAB_OK;
