@@ -79,8 +79,10 @@ struct AdjDesc {
   const float* src;      // MODE 1: (nInst, H, W)
   const float* dst;      // MODE 1: (nInst, H, W)
   uint32_t* sig;         // optional (nInst, nPts): hash of every cell the forward sweep looked up
-  double* ckpt;          // (nInst, nT, nPts, 2) workspace: start points of the steps (calc_T map: of the events)
-  uint16_t* event;       // calc_T map: (nInst, nT, nPts) workspace, the events (adj_event)
+  double* ckpt;          // (nInst, nT, ckPts, 2) workspace: start points of the steps (calc_T map: of the events)
+  uint16_t* event;       // calc_T map: (nInst, nT, ckPts) workspace, the events (adj_event)
+  int64_t blk0, nBlk;    // this launch's first block of each instance's nBlk
+  int64_t ckPts;         // points of the launch's blocks
   double* partial;       // (nInst, blocks per instance, NG*nC*6 + 2): tables, loss, redone steps
   double h;
   int nT, nS;
@@ -122,6 +124,7 @@ __device__ __forceinline__ int adj_steps(int ev) { return ev >> 10; }
 // 8 718, 10 709; more do not fit the registers), and runs between two redo
 // phases of the forward sweep (5 the same, 10: 755).
 constexpr int kAdjRun = 10;
+static_assert(kAdjRun < 64, "six bits of adj_event");
 constexpr int kAdjSegs = 3;
 
 __device__ __forceinline__ uint32_t sig_mix(uint32_t s, int c) { return s * 0x9E3779B1u + (uint32_t)(c + 1); }
@@ -206,8 +209,8 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
   // domain corner (a pixel that can redo most of its steps: the longest
   // chain of trips), then start before any instance's other blocks
   const int inst = D.inst_major ? (int)blockIdx.x : (int)blockIdx.y;
-  const int64_t blk = D.inst_major ? (int64_t)blockIdx.y : (int64_t)blockIdx.x;
-  const int64_t nblk = D.inst_major ? (int64_t)gridDim.y : (int64_t)gridDim.x;
+  const int64_t bl = D.inst_major ? (int64_t)blockIdx.y : (int64_t)blockIdx.x;  // in this launch
+  const int64_t blk = D.blk0 + bl;
   const int nC = D.nC, NT = nC * 6;
   const int nW = blockDim.x >> 6, wave = threadIdx.x >> 6;
   double* At = lds;
@@ -234,7 +237,7 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
     // the point's index in the caller's arrays: idx, or in MODE 1 with tiles
     // the pixel of lane idx & 63 in 8 x 8 tile idx >> 6 (neighbouring pixels
     // cross facets at about the same steps, so fewer of a wave's steps have
-    // a redone lane; the checkpoints stay indexed by idx)
+    // a redone lane; the checkpoints stay in the order of idx)
     int64_t pix = idx;
     if (MODE == 1 && D.tile8) {
       const int64_t t = idx >> 6;
@@ -249,8 +252,9 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
       p[0] = (double)(pix % D.W);
       p[1] = (double)(pix / D.W);
     }
-    double* ck = D.ckpt + (int64_t)inst * nT * nPts * 2;
-    uint16_t* evs = FWD ? D.event + (int64_t)inst * nT * nPts : nullptr;
+    const int64_t ckPts = D.ckPts, cp = bl * blockDim.x + threadIdx.x;  // the point's place in the workspace
+    double* ck = D.ckpt + (int64_t)inst * nT * ckPts * 2;
+    uint16_t* evs = FWD ? D.event + (int64_t)inst * nT * ckPts : nullptr;
     uint32_t sg = 0;
     // the cell of p, carried: an accepted step ends in the cell it started
     // in, and each substep looks up the cell of its end point
@@ -258,13 +262,13 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
     int nev = 0;  // events logged
     if (FWD) {
       // Forward sweep of calc_T's map in the two phases of `advance`; logged
-      // are events, each with its start point: up to NSM accepted steps, or
+      // are events, each with its start point: up to kAdjRun accepted steps, or
       // one redone step.
       const bool has_sig = D.sig != nullptr;
       auto log_start = [&](const double* q) {
-        *reinterpret_cast<double2*>(ck + ((int64_t)nev * nPts + idx) * 2) = make_double2(q[0], q[1]);
+        *reinterpret_cast<double2*>(ck + ((int64_t)nev * ckPts + cp) * 2) = make_double2(q[0], q[1]);
       };
-      auto log_event = [&](int cell, int n) { evs[(int64_t)nev++ * nPts + idx] = adj_event(cell, n); };
+      auto log_event = [&](int cell, int n) { evs[(int64_t)nev++ * ckPts + cp] = adj_event(cell, n); };
       int t = 0, cool = 0;
       for (;;) {
         const uint64_t todo = ballot(t < nT);
@@ -341,8 +345,8 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
       }
     } else {  // calc_T_simple's map: a checkpoint a time step, every step nS substeps
       for (int k = 0; k < nT; k++) {
-        ck[((int64_t)k * nPts + idx) * 2] = p[0];
-        ck[((int64_t)k * nPts + idx) * 2 + 1] = p[1];
+        ck[((int64_t)k * ckPts + cp) * 2] = p[0];
+        ck[((int64_t)k * ckPts + cp) * 2 + 1] = p[1];
         nredo++;
         for (int j = 0; j < nS; j++) {
           sg = sig_mix(sg, c);
@@ -451,9 +455,9 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
       int ev = 0;
       auto load_event = [&]() {
         if (e >= 0) {
-          const int64_t pt = tail ? idx - lane + L : idx;
-          q2 = *reinterpret_cast<const double2*>(ck + ((int64_t)e * nPts + pt) * 2);
-          ev = evs[(int64_t)e * nPts + pt];
+          const int64_t pt = tail ? cp - lane + L : cp;
+          q2 = *reinterpret_cast<const double2*>(ck + ((int64_t)e * ckPts + pt) * 2);
+          ev = evs[(int64_t)e * ckPts + pt];
         }
       };
       load_event();
@@ -563,12 +567,12 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
       }
     } else {  // calc_T_simple's map: every step is nS substeps, the same on every lane
       // (the checkpoint of the step before is loaded while a step is processed)
-      double qn[2] = {ck[((int64_t)(nT - 1) * nPts + idx) * 2], ck[((int64_t)(nT - 1) * nPts + idx) * 2 + 1]};
+      double qn[2] = {ck[((int64_t)(nT - 1) * ckPts + cp) * 2], ck[((int64_t)(nT - 1) * ckPts + cp) * 2 + 1]};
       for (int k = nT - 1; k >= 0; k--) {
         const double q[2] = {qn[0], qn[1]};
         if (k > 0) {
-          qn[0] = ck[((int64_t)(k - 1) * nPts + idx) * 2];
-          qn[1] = ck[((int64_t)(k - 1) * nPts + idx) * 2 + 1];
+          qn[0] = ck[((int64_t)(k - 1) * ckPts + cp) * 2];
+          qn[1] = ck[((int64_t)(k - 1) * ckPts + cp) * 2 + 1];
         }
         redone_step(q);
       }
@@ -581,7 +585,7 @@ __global__ void __launch_bounds__(256, 4) k_adjoint2d(AdjDesc D) {
   const double nr = block_sum((double)nredo, red);
   __syncthreads();
   // the block's tables: its waves' tables summed in wave order
-  double* out = D.partial + ((int64_t)inst * nblk + blk) * (NG * NT + 2);
+  double* out = D.partial + ((int64_t)inst * D.nBlk + blk) * (NG * NT + 2);
   for (int i = threadIdx.x; i < NG * NT; i += blockDim.x) {
     double s = 0.0;
     for (int w = 0; w < nW; w++) s += Gall[(size_t)w * NG * NT + i];

@@ -656,8 +656,11 @@ int ensure_ws(cpab_ctx* ctx, size_t bytes) {
     ctx->ws_bytes = 0;
   }
   hipError_t e = hipMalloc(&ctx->ws, bytes);
-  if (e != hipSuccess) return fail(ctx, CPAB_ERR_NOMEM, "hipMalloc(%zu) for the adjoint workspace: %s", bytes,
-                                   hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // (or the next launch's check would report it)
+    ctx->ws = nullptr;
+    return fail(ctx, CPAB_ERR_NOMEM, "hipMalloc(%zu) for the adjoint workspace: %s", bytes, hipGetErrorString(e));
+  }
   ctx->ws_bytes = bytes;
   return CPAB_OK;
 }
@@ -698,10 +701,21 @@ int adjoint2d(cpab_ctx* ctx, int mode, int tess, int nC, int nInst, int64_t nPts
   const int block = 64 * waves;
   const int64_t nbx = (nPts + block - 1) / block;
   if (nbx > 0x7fffffffLL) return fail(ctx, CPAB_ERR_ARG, "too many points");
-  const size_t ck = (size_t)nInst * nT * nPts * 2, pa = (size_t)nInst * nbx * (NG * NT + 2);
-  const size_t gt = fwd ? (size_t)nInst * NT : 0;
-  const size_t rb = fwd ? ((size_t)nInst * nT * nPts + 3) / 4 : 0;  // the events, 16 bits each
-  if ((r = ensure_ws(ctx, (ck + pa + gt + rb) * sizeof(double)))) return r;
+  const size_t pa = (size_t)nInst * nbx * (NG * NT + 2), gt = fwd ? (size_t)nInst * NT : 0;
+  // The workspace of a launch: 16 bytes a step and point, and 2 for the events
+  // of the calc_T map.  Where that much memory is not to be had, the blocks are
+  // run in parts that share a smaller one (the same sums).
+  int64_t nb = nbx, ckPts;
+  size_t ck, ev;
+  for (;;) {
+    ckPts = std::min(nPts, nb * block);
+    ck = (size_t)nInst * nT * ckPts * 2;
+    ev = fwd ? ((size_t)nInst * nT * ckPts + 3) / 4 : 0;
+    r = ensure_ws(ctx, (ck + pa + gt + ev) * sizeof(double));
+    if (r != CPAB_ERR_NOMEM || nb == 1) break;
+    nb = (nb + 1) / 2;
+  }
+  if (r) return r;
   AdjDesc D{};
   D.nInst = nInst;
   D.nC = nC;
@@ -719,6 +733,8 @@ int adjoint2d(cpab_ctx* ctx, int mode, int tess, int nC, int nInst, int64_t nPts
   D.ckpt = ctx->ws;
   D.partial = ctx->ws + ck;
   D.event = fwd ? reinterpret_cast<uint16_t*>(ctx->ws + ck + pa + gt) : nullptr;
+  D.ckPts = ckPts;
+  D.nBlk = nbx;
   const bool ns10 = nS <= 10;  // the substep starts of a redone step in 10 registers pairs, else 16
   D.h = dt / (double)nS;
   D.nT = nT;
@@ -728,9 +744,9 @@ int adjoint2d(cpab_ctx* ctx, int mode, int tess, int nC, int nInst, int64_t nPts
   // instances' first blocks (the domain corner's long chain) first, while
   // the blocks per instance fit the grid's y dimension
   D.inst_major = nbx <= 65535 ? 1 : 0;
-  const dim3 grid = D.inst_major ? dim3((unsigned)nInst, (unsigned)nbx) : dim3((unsigned)nbx, (unsigned)nInst);
   hipEvent_t a = nullptr, b = nullptr;
   if ((r = prof_begin(ctx, &a, &b))) return r;
+  int launches = 0;
 #define ADJ_LAUNCH4(T_, P_, M_, F_)                                        \
   do {                                                                     \
     if (ns10) {                                                            \
@@ -753,18 +769,22 @@ int adjoint2d(cpab_ctx* ctx, int mode, int tess, int nC, int nInst, int64_t nPts
     if (mode == 0) ADJ_LAUNCH3(T_, P_, 0);   \
     else ADJ_LAUNCH3(T_, P_, 1);             \
   } while (0)
-  if (tess == TESS_I) {
-    if (pow2) ADJ_LAUNCH(TESS_I, true);
-    else ADJ_LAUNCH(TESS_I, false);
-  } else {
-    if (pow2) ADJ_LAUNCH(TESS_II, true);
-    else ADJ_LAUNCH(TESS_II, false);
+  for (D.blk0 = 0; D.blk0 < nbx; D.blk0 += nb, launches++) {
+    const unsigned part = (unsigned)std::min(nb, nbx - D.blk0);
+    const dim3 grid = D.inst_major ? dim3((unsigned)nInst, part) : dim3(part, (unsigned)nInst);
+    if (tess == TESS_I) {
+      if (pow2) ADJ_LAUNCH(TESS_I, true);
+      else ADJ_LAUNCH(TESS_I, false);
+    } else {
+      if (pow2) ADJ_LAUNCH(TESS_II, true);
+      else ADJ_LAUNCH(TESS_II, false);
+    }
   }
 #undef ADJ_LAUNCH
 #undef ADJ_LAUNCH3
 #undef ADJ_LAUNCH4
   HIP_OK(ctx, hipGetLastError());
-  if ((r = prof_end(ctx, a, b))) return r;
+  if ((r = prof_end(ctx, a, b, launches))) return r;
   double* gradT = fwd ? ctx->ws + ck + pa : nullptr;
   hipLaunchKernelGGL(k_adj_reduce, dim3((unsigned)((NG * NT + 2 + 63) / 64), (unsigned)nInst), dim3(64), 0, ctx->stream,
                      D.partial, (int)nbx, NT, NG, gradA, gradT, loss, nredo);

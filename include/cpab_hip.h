@@ -123,7 +123,8 @@ int cpab_calc_grad_theta(cpab_ctx *ctx, int dim, int tess, int nC, const double 
  * cotangents lam (nInst, nPts, 2) of the end points, gradA (nInst, nC, 6) =
  * sum_x lam(x)^T dT(x)/dA, A the integrated (signed) tables As (nInst, nC, 6).
  * dtheta follows as B^T gradA (times the sign).  One checkpoint per time step
- * in a library workspace (16 * nTimeSteps bytes per point); the substeps are
+ * in a library workspace (16 * nTimeSteps bytes per point, in parts of the
+ * points where there is no memory for all of them); the substeps are
  * recomputed.  nStepsODE <= 16.  The tables and per-wave gradient tables
  * live in LDS: nC up to 1706 here, 853 for the calc_T map below
  * (CPAB_ERR_UNSUPPORTED beyond).  pos_out (optional): the end points. */
@@ -152,8 +153,8 @@ int cpab_ssd_grad2d(cpab_ctx *ctx, int tess, int nC, int nInst, const double *As
  * signed tables (nInst, nC, 6).  gradA = sum_x lam(x)^T dT(x)/dAs, through
  * the Trel steps (the adjoint of the Frechet derivative of expm) and the RK2
  * substeps.  The additions follow a fixed order: gradA is the same bit for bit
- * on every run.  Same checkpoint workspace and limits as
- * cpab_calc_T_simple_vjp. */
+ * on every run.  Workspace 18 * nTimeSteps bytes per point, else as
+ * cpab_calc_T_simple_vjp's; the same limits. */
 int cpab_calc_T_vjp(cpab_ctx *ctx, int tess, int nC, int nInst, const double *pos0,
                     const double *lam, const double *Trels, const double *As, double dt,
                     int nTimeSteps, int nStepsODE, int64_t nPts, int nC0, int nC1, double inc_x,
