@@ -101,7 +101,7 @@ __device__ __forceinline__ int axis_box(double p, int nC, double inc, double rin
 // One clamped axis of the type I lookups: the box index (mymin of
 // (p0 - xmod) / inc, calc_2Dto2D.cu:20-22) and the in-box coordinate: frac =
 // xmod / inc (POW2), or the remainder xmod itself, whose division the caller
-// puts off (simplex_frac).
+// puts off (triangle_of, cell3).
 template <bool POW2>
 __device__ __forceinline__ int axis_simplex(double p0, int nC, double inc, double rinc, double& frac) {
   int i;

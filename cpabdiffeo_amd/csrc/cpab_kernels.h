@@ -12,7 +12,7 @@
 //                  a wave step together while their points stay in their
 //                  cells and redo steps together when they have left them
 //                  (`advance`), and lanes that finish take the next points
-//                  of their wave's range.  Per point, the sequence of IEEE
+//                  of their block's range.  Per point, the sequence of IEEE
 //                  operations is the reference's.
 //  * k_simple      calc_T_simple (calc_2Dto2D.cu:412-445).
 //  * k_velocity    calc_v (calc_2Dto2D.cu:561-602).
@@ -765,7 +765,7 @@ __device__ __forceinline__ void advance_lockstep(double* p, int& c, int& k, int&
 // Lane state: p (current point), c (cell of p), t (steps done).  solveODE
 // recomputes cell(p) at the top of every substep; here it is the lookup at
 // the end of the previous one, of the same p: same value.  Lanes retire and
-// take the next points of the wave's range between calls of `advance`.
+// take the next points of the block's range between calls of `advance`.
 //
 // Processing index i -> point index of n points that form a row-major grid
 // of row length w: bands of r = 1 << lr rows are walked in tiles of r rows and
@@ -994,10 +994,10 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5)))
 // substep; no branch between the columns, whose LDS reads each stalled the
 // wave when the rows were read every substep (and staged: now a wave reads
 // rows on the ~1/4 of its substeps in which some point changes cell, and from
-// LDS that measured the same).  128 x 128 grid, 62 columns: 1.86 -> 1.63 ms
+// LDS that measured the same).  128 x 128 grid, 62 columns: 1.86 -> 1.55 ms
 // (0.25 of it the corner's pixel, which changes cell every substep); 16 384
 // random points 2.79 -> 1.35 ms (28 T instructions/s of the 39 that two waves
-// a SIMD can issue), 2 000: 1.55 -> 0.31, 500: 1.55 -> 0.20.
+// a SIMD can issue), 2 000: 1.55 -> 0.30, 500: 1.55 -> 0.20.
 template <int DIM, int TESS, bool POW2, int JC>
 __global__ void __launch_bounds__(256, 2)
     k_grad_theta(const double* __restrict__ pos0, double* __restrict__ pos, const double* __restrict__ As,

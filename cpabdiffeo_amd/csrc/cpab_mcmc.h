@@ -70,55 +70,53 @@ namespace cpab {
 // the cell being wave-uniform here, measured 1-2 % slower than LDS.)  Same
 // schedule and IEEE operations as `trip`.  Runs until t >= tb and leaves row
 // consistent with (c, k).
-template <int DIM, int TESS, bool POW2>
+template <int TESS, bool POW2>
 __device__ __forceinline__ int lone_cell(const double* y, const Geom& g) {
-  if (DIM == 2 && TESS == TESS_I && POW2) return cell2_flat(y, g);
-  return cell_of<DIM, TESS, POW2>(y, g);
+  if (TESS == TESS_I && POW2) return cell2_flat(y, g);
+  return cell2<TESS, POW2>(y, g);
 }
 
-template <int DIM, int TESS, bool POW2>
+template <int TESS, bool POW2>
 __device__ __forceinline__ void lone_trips(double* p, int& c, int& k, int& t, int tb, const double*& row, int& nfb,
                                            const double* Ttab, const double* Atab, double h, int nS,
                                            const Geom& g) {
-  constexpr int NE = DIM * (DIM + 1);
   const double hh = h * 0.5;  // as in `trip`
   while (t < tb) {
     const double* r = row;
-    double y[DIM];
-    affine<DIM>(y, r, p);
+    double y[2];
+    affine<2>(y, r, p);
     if (k == 0) {  // Trel proposal
-      const int cy = lone_cell<DIM, TESS, POW2>(y, g);
+      const int cy = lone_cell<TESS, POW2>(y, g);
       if (cy == c) {
-#pragma unroll
-        for (int d = 0; d < DIM; d++) p[d] = y[d];
+        p[0] = y[0];
+        p[1] = y[1];
         t++;
       } else {
         nfb++;
         if (nS > 0) {
           k = nS;
-          row = Atab + mul24(c, NE);
+          row = Atab + mul24(c, 6);
         } else {
           t++;
         }
       }
     } else {  // one RK2 midpoint substep
-      double m[DIM];
-#pragma unroll
-      for (int d = 0; d < DIM; d++) m[d] = p[d] + hh * y[d];
-      affine<DIM>(y, r, m);
-#pragma unroll
-      for (int d = 0; d < DIM; d++) y[d] = p[d] + y[d] * h;
-      const int cy = lone_cell<DIM, TESS, POW2>(y, g);
-#pragma unroll
-      for (int d = 0; d < DIM; d++) p[d] = y[d];
+      double m[2];
+      m[0] = p[0] + hh * y[0];
+      m[1] = p[1] + hh * y[1];
+      affine<2>(y, r, m);
+      y[0] = p[0] + y[0] * h;
+      y[1] = p[1] + y[1] * h;
+      const int cy = lone_cell<TESS, POW2>(y, g);
+      p[0] = y[0];
+      p[1] = y[1];
       const bool done = --k == 0;
-      if (done | (cy != c)) row = (done ? Ttab : Atab) + mul24(cy, NE);
+      if (done | (cy != c)) row = (done ? Ttab : Atab) + mul24(cy, 6);
       c = cy;
       if (done) t++;
     }
   }
 }
-
 
 struct Philox {
   uint32_t x0, x1, x2, x3;
@@ -792,7 +790,7 @@ __global__ void __launch_bounds__(BLOCK) k_mcmc_step(McmcDesc D, int init) {
         }
         if (!active || t >= nT) continue;
         if (__popcll(__builtin_amdgcn_read_exec()) == 1) {  // one lane left: it loops on its own
-          lone_trips<2, TESS, POW2>(p, c, k, t, tb, row, nfb, Ttab, Atab, h, nS, g);
+          lone_trips<TESS, POW2>(p, c, k, t, tb, row, nfb, Ttab, Atab, h, nS, g);
           continue;
         }
         for (;;) {  // two trips per iteration (written out: the compiler does not unroll around a ballot)
