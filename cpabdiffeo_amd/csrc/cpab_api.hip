@@ -930,9 +930,15 @@ int batch_launch(cpab_batch* b, hipStream_t s, const cpab_batch_sched& q, const 
   int grid = ctx->n_cu * per_cu;
   const int64_t chunks = ((int64_t)b->nTiles + q.chunk - 1) / q.chunk;
   if (grid > chunks) grid = (int)chunks;
+  // The fewest tiles of a grab.  One, so that blocks end together; but a grab is
+  // ~70 ns of the one counter, so where a tile is a microsecond or two of its
+  // block and the chunks are many, the whole chunk (300 instances of 30 000 1D
+  // points, tiles of 1 024, chunk 8, 10 steps of 3: one 681 us, the chunk 246;
+  // batches of fewer tiles are up to three times slower with the chunk).
+  const bool brief = (int64_t)q.tile * nT < (1 << 15) && chunks >= 4 * (int64_t)ctx->n_cu;
   hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, s, b->queue);
-  hipLaunchKernelGGL(k, dim3(grid), dim3(q.block), lds, s, b->d_inst, b->d_tiles, b->nTiles, q.chunk, b->queue,
-                     tables, pos0, out, h, nT, nS, nfb, sort_off);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(q.block), lds, s, b->d_inst, b->d_tiles, b->nTiles, q.chunk,
+                     brief ? q.chunk : 1, b->queue, tables, pos0, out, h, nT, nS, nfb, sort_off);
   HIP_OK(ctx, hipGetLastError());
   return CPAB_OK;
 }

@@ -142,7 +142,7 @@ __device__ void tile_bucket_order(const double* __restrict__ pos0, int64_t begin
 template <int DIM, int TESS, bool POW2>
 __global__ void __launch_bounds__(1024)
     k_integrate_batch(const BatchInst* __restrict__ insts, const BatchTile* __restrict__ tiles, int nTiles, int chunk,
-                      unsigned int* __restrict__ queue, const double* __restrict__ tables,
+                      int least, unsigned int* __restrict__ queue, const double* __restrict__ tables,
                       const double* __restrict__ pos0, double* __restrict__ out, double h, int nT, int nS,
                       int32_t* __restrict__ nfb_out, int sort_off) {
   constexpr int NE = DIM * (DIM + 1);
@@ -157,13 +157,13 @@ __global__ void __launch_bounds__(1024)
     __syncthreads();  // every wave is done with the previous chunk's s_t0
     if (threadIdx.x == 0) {
       // `chunk` tiles at a time while each block has four such grabs ahead of
-      // it, then fewer, in the end one (256 instances, tiles of 16 384, chunk
+      // it, then fewer, in the end `least` (256 instances, tiles of 16 384, chunk
       // 4: 2 400 tiles are 2.3 grabs for each of 256 blocks, and the launch
       // waited for those that took three)
       const unsigned int seen = __hip_atomic_load(queue, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const int left = seen < (unsigned int)nTiles ? nTiles - (int)seen : 0;
       int k = left / (4 * (int)gridDim.x);
-      k = k < 1 ? 1 : (k > chunk ? chunk : k);
+      k = k < least ? least : (k > chunk ? chunk : k);
       s_t0 = (int)atomicAdd(queue, (unsigned int)k);
       s_t1 = s_t0 + k;
     }
