@@ -844,8 +844,11 @@ __device__ __forceinline__ void integrate_points(int64_t begin, int n, int* curs
   // a grid's tiles are 64 neighbouring points that need similar work, so a
   // wave takes one after another (2048 x 2048 points: 750 -> 610 us); other
   // waves take the next points as soon as kRefill lanes are free (256 batched
-  // instances, 8 instead of 16: 14.3 -> 13.9 ms, 32: 16.7; 64: 15.3)
-  const int refill = gord.w > 0 ? 64 : kRefill;
+  // instances, 8 instead of 16: 14.3 -> 13.9 ms, 32: 16.7; 64: 15.3).  Trajectories
+  // larger than the cache: a wave's points all start together, or the others
+  // would wait for the new ones (kSpread).
+  const bool far = MODE == 1 && nT * nPts > kCacheBytes / (8 * DIM);
+  const int refill = gord.w > 0 || far ? 64 : kRefill;
   double p[DIM];
 #pragma unroll
   for (int d = 0; d < DIM; d++) p[d] = 0.0;
@@ -899,8 +902,7 @@ __device__ __forceinline__ void integrate_points(int64_t begin, int n, int* curs
                                               MODE == 1 ? out + my * DIM : nullptr, nPts);
     } else if (MODE == 1 || (active && t < nT)) {  // (calc_trajectory's compares the lanes' steps: all of them call it)
       advance<DIM, TESS, POW2, MODE>(p, c, t, nT, nfb, Ttab, Atab, h, nS, g, more, refill,
-                                     MODE == 1 ? out + my * DIM : nullptr, nPts,
-                                     MODE == 1 && nT * nPts > kCacheBytes / (8 * DIM));
+                                     MODE == 1 ? out + my * DIM : nullptr, nPts, far);
     }
   }
 }

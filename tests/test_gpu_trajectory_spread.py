@@ -1,7 +1,8 @@
 """calc_trajectory with more rows than the 256 MiB cache holds.
 
-There a lane of a wave stays within 16 steps of the wave's last one.  Just
-above that size, with points at rest (on walls), calm ones and ones that change
+There a lane of a wave stays within 16 steps of the wave's last one, and a
+wave's points all start together.  Just above that size, a point and two points
+a lane, with points at rest (on walls), calm ones and ones that change
 cell at most steps in each wave: every row against the oracle, bit for bit
 (cpab/gpu/calc_2Dto2D.cu:499-556)."""
 import numpy as np
@@ -13,11 +14,12 @@ from test_gpu_simple_walls import tables
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dim,tess,nCs,extent", [(1, "II", (8,), (1.0,)), (2, "I", (4, 4), (1.0, 1.0)),
-                                                 (2, "II", (5, 3), (640.0, 480.0)), (3, "I", (2, 2, 2), (1.0, 1.0, 1.0))])
-def test_rows_equal_the_oracle(gpu, orc, dim, tess, nCs, extent):
+@pytest.mark.parametrize("dim,tess,nCs,extent,nT", [
+    (1, "II", (8,), (1.0,), 240), (2, "I", (4, 4), (1.0, 1.0), 240), (2, "II", (5, 3), (640.0, 480.0), 240),
+    (3, "I", (2, 2, 2), (1.0, 1.0, 1.0), 240), (1, "II", (8,), (1.0,), 60), (2, "I", (3, 5), (1.0, 1.0), 28)])
+def test_rows_equal_the_oracle(gpu, orc, dim, tess, nCs, extent, nT):
     torch = gpu
-    nT, nS, dt = 240, 3, 1.0 / 240
+    nS, dt = 3 if nT > 33 else 4, 1.0 / nT
     n = (256 << 20) // (8 * dim * nT) + 70
     print("[gpu] trajectory of", n, "points", dim, tess, nCs, flush=True)
     rng = np.random.default_rng(23)
