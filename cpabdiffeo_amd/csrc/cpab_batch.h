@@ -235,7 +235,8 @@ __global__ void __launch_bounds__(1024)
   // sort_off > 0: runs of up to sort_cap points in an order by position (tile_bucket_order)
   unsigned int* hist = reinterpret_cast<unsigned int*>(lds + sort_off);
   uint16_t* idx = reinterpret_cast<uint16_t*>(hist + kBucketMax);
-  const double* cur = nullptr;  // Trels in LDS (block-uniform)
+  const double *cur = nullptr, *cur_as = nullptr;  // the tables in LDS (block-uniform)
+  int cur_nC = 0;
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -254,9 +255,8 @@ __global__ void __launch_bounds__(1024)
     for (int t = t0; t < t1;) {
       const WorkItem& it = items[t];
       const int nC = it.nC;
-      const double* tr = it.trels;
-      if (tr != cur) {
-        const double* sa = it.as;
+      const double *tr = it.trels, *sa = it.as;
+      if (tr != cur || sa != cur_as || nC != cur_nC) {
         __syncthreads();
         for (int i = threadIdx.x; i < nC * NE; i += blockDim.x) {
           lds[i] = tr[i];
@@ -264,6 +264,8 @@ __global__ void __launch_bounds__(1024)
         }
         __syncthreads();
         cur = tr;
+        cur_as = sa;
+        cur_nC = nC;
       }
       const Geom g = it.g;
       const double* pos0 = it.pos0;
@@ -271,7 +273,7 @@ __global__ void __launch_bounds__(1024)
       int64_t end = it.end;
       for (t++; t < t1; t++) {  // the items that go on where this one ends
         const WorkItem& nx = items[t];
-        if (nx.trels != tr || nx.as != it.as || nx.pos0 != pos0 || nx.out != it.out || nx.begin != end ||
+        if (nx.trels != tr || nx.as != sa || nx.pos0 != pos0 || nx.out != it.out || nx.begin != end ||
             nx.g.nC0 != g.nC0 || nx.g.nC1 != g.nC1 || nx.g.nC2 != g.nC2 || nx.g.inc_x != g.inc_x ||
             nx.g.inc_y != g.inc_y || nx.g.inc_z != g.inc_z || nx.end - it.begin > most)
           break;
