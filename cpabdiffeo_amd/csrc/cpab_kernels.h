@@ -541,7 +541,7 @@ constexpr int kTrips = 2;  // trips in lockstep between two looks at the lanes t
 // 30 steps of 10 take 0.60 of the time of an older lockstep kernel (median of
 // 36 calls), lockstep 0.73; 100 steps of 4 0.63 and 0.75.
 __host__ __device__ constexpr bool lockstep_pays(int dim, int nT, int nS) {
-  return (int64_t)nT * nS <= 100 || (dim == 3 && nT < 64);
+  return (int64_t)nT * (nS > 0 ? nS : 1) <= 100 || (dim == 3 && nT < 64);
 }
 
 // The point at the domain's corner (0, 0).  With zero velocity on the walls

@@ -20,7 +20,7 @@ from test_gpu_simple_walls import CASES, points, tables
 
 pytestmark = pytest.mark.gpu
 
-STEPS = [(0, 5), (1, 5), (3, 33), (10, 10), (100, 1), (101, 1), (10, 11), (7, 0), (2, 60), (40, 4), (63, 4), (64, 4), (120, 10)]
+STEPS = [(0, 5), (1, 5), (3, 33), (10, 10), (100, 1), (101, 1), (10, 11), (7, 0), (150, 0), (2, 60), (40, 4), (63, 4), (64, 4), (120, 10)]
 
 
 @pytest.mark.parametrize("dim,tess,nCs,extent", CASES)
